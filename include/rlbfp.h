@@ -210,6 +210,16 @@ int rl_ln_modulate(const uint16_t *x, int64_t ldx, const void *branch, int32_t b
                    uint8_t *a_packed, int32_t a_order, uint16_t *a_deq, int64_t ld_a, int64_t M, int64_t D,
                    void *stream);
 
+/* rl_ln_modulate on the stream formats that the artifact itself takes (run_ln.ln_pack_x / ln_pack_br,
+ * redline/run_ln.py:28-35): x and x_out hold bf16 values in the C-stream element order c_layout_atb(., 128, 128) of
+ * (M, D), the branch (may be NULL) bf16 or bfp16 blocks in that order, and a_packed receives y as bfp16 in
+ * RL_ORDER_A_LAYOUT. Same values as rl_ln_modulate (x' bit for bit; the row sums run in another order). x_out may equal
+ * x; the outputs must not overlap the inputs otherwise. M % 512 == 0, D % 1024 == 0, D <= 8192; every pointer 16-byte
+ * aligned (a packed branch 4-byte). Same reference interface as rl_ln_modulate. */
+int rl_ln_modulate_stream(const uint16_t *x, const void *branch, int32_t br_fmt, const uint16_t *params,
+                          int64_t split_row, int32_t norm, uint16_t *x_out, uint8_t *a_packed, int64_t M, int64_t D,
+                          void *stream);
+
 /* ---- QKV post: the QKV GEMM output -> attention Q / K / V --------------------------------------------------------
  * C (M, 3 * heads * 128) bf16 row major (ldc): per token row the q, k and v columns of `heads` heads of 128 dims.
  * Per head and token row, in fp32:

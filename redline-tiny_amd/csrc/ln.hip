@@ -301,6 +301,191 @@ static int launch_upto(int nb, const LnArgs& a, hipStream_t st) {
   }
 }
 
+// ---- the same op on streams: x, the branch and x' in the C-stream order, A packed in the A layout --------------------
+//
+// Workgroup = 8 rows (one br half of a 16-row band), 512 threads; thread f + 512 j takes the 8-value block (row rib =
+// f & 7, 16-byte column blocks in stream order), so that 16 consecutive lanes hold 16 consecutive blocks of the
+// stream: a wave's load or store is four runs of 256 bytes (bf16) or 144 bytes (packed). The two halves of a band
+// share their cache lines; xcd_remap puts them on one XCD. A row's values are spread over the lanes of equal rib of
+// all 8 waves, so the mean and the variance take a wave reduction, an LDS exchange and a barrier each.
+// HBM-bound: 2 + 9/8 (or 2) bytes read and 2 + 9/8 written per value, once. 4096 x 4096 with a packed branch (105 MB)
+// replaces index-tensor permutations of x and x', a dequantize pass, the row-major kernel and a copy (1063 us);
+// it takes 28 us (3.7 TB/s). All of a row's loads are issued before the first use; 8 rows x D values stay in registers
+// as bf16 pairs (32 VGPRs at D = 4096: the 512 workgroups of 4096 rows are all resident, 2 per CU).
+constexpr int kLsThreads = 512, kLsRows = 8;
+
+struct LnStreamArgs {
+  const uint16_t* x;
+  const void* br;
+  const uint16_t* params;
+  int64_t split_row;
+  int32_t norm;
+  uint16_t* x_out;
+  uint8_t* a_packed;
+  int32_t D;
+};
+
+// Sum over the 8 lanes of equal lane & 7, every lane getting the result
+__device__ __forceinline__ float sum_rib(float v) {
+  v += dpp_f<0x128>(v);  // row_ror:8
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// NB = blocks per thread (D / 512); BR: 0 no branch, 1 bf16, 2 packed
+template <int NB, int BR>
+__global__ __launch_bounds__(kLsThreads, NB <= 8 ? 4 : 2) void ln_stream_kernel(LnStreamArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t stage[];
+  __shared__ float red[2][kLsThreads / 64][kLsRows];
+  const int tid = threadIdx.x, lane = tid & 63, rib = tid & 7;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int D = a.D;
+  const int64_t r0 = (int64_t)xcd_remap(blockIdx.x, gridDim.x) * kLsRows;
+  const uint16_t* prm = a.params + (r0 + rib < a.split_row ? 2 * D : 0);  // [g | sc] row
+  // stream block of item j: tile column c128 = 4 j + tid / 128 (8192 blocks apart), then sbc, br, bc, rib
+  const int sbc = (tid >> 4) & 7, bc = (tid >> 3) & 1;
+  const int64_t blk0 = ((r0 >> 9) * (D >> 7) + (tid >> 7)) * 8192 + ((r0 >> 7) & 3) * 2048 + ((r0 >> 4) & 7) * 256 +
+                       sbc * 32 + ((r0 >> 3) & 1) * 16 + bc * 8 + rib;
+  const int cb0 = (tid >> 7) * 16 + sbc * 2 + bc;  // column block; + 64 j
+  constexpr int kStep = 4 * 8192;                  // stream blocks between items j and j + 1
+
+  u32x4 v[NB];
+  float s = 0.f;
+  constexpr int kC = NB <= 8 ? NB : (NB + 1) / 2;  // loads in flight: whole rows, or two chunks above D = 4096
+#pragma unroll
+  for (int j0 = 0; j0 < NB; j0 += kC) {
+    u32x4 xr[kC], brw[kC];
+#pragma unroll
+    for (int c = 0; c < kC; c++) {
+      if (j0 + c >= NB) break;
+      const int64_t blk = blk0 + (int64_t)(j0 + c) * kStep;
+      xr[c] = *reinterpret_cast<const u32x4*>(a.x + blk * 8);
+      if constexpr (BR == 1) brw[c] = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.br) + blk * 8);
+      if constexpr (BR == 2) {
+        // the window of a stream's last block (odd index) ends with the block
+        const Window w = load_window(static_cast<const uint8_t*>(a.br), blk * 9);
+        brw[c] = u32x4{w.w0, w.w1, w.w2, 0u};
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < kC; c++) {
+      const int j = j0 + c;
+      if (j >= NB) break;
+      const int64_t blk = blk0 + (int64_t)j * kStep;
+      u32x4 xw = xr[c];
+      if constexpr (BR != 0) {
+        float xf[8], gf[8], bf[8];
+        unpack8(xr[c], xf);
+        unpack8(*reinterpret_cast<const u32x4*>(prm + (cb0 + 64 * j) * 8), gf);
+        if constexpr (BR == 1) {
+          unpack8(brw[c], bf);
+        } else {
+          const uint32_t o = (uint32_t)(rib & 3);  // (9 * blk) % 4: blk % 4 == rib % 4
+          const uint32_t lo = __builtin_amdgcn_alignbyte(brw[c].y, brw[c].x, o);
+          const uint32_t hi = __builtin_amdgcn_alignbyte(brw[c].z, brw[c].y, o);
+          const int sh = (int)(lo & 0xFFu) - 133;
+          const int32_t q[8] = {(int8_t)(lo >> 8), (int8_t)(lo >> 16), (int8_t)(lo >> 24), (int8_t)hi,
+                                (int8_t)(hi >> 8), (int8_t)(hi >> 16), (int8_t)(hi >> 24),
+                                (int8_t)(brw[c].z >> (8 * o))};
+#pragma unroll
+          for (int e = 0; e < 8; e++) bf[e] = __builtin_amdgcn_ldexpf((float)q[e], sh);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          xw[e] = pack_bf16_rne(fmaf(gf[2 * e], bf[2 * e], xf[2 * e]), fmaf(gf[2 * e + 1], bf[2 * e + 1], xf[2 * e + 1]));
+      }
+      const bf16x2 one = {(__bf16)1.0f, (__bf16)1.0f};
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const uint32_t w = xw[e];
+        s = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w), one, s, false);
+      }
+      v[j] = xw;
+      *reinterpret_cast<u32x4*>(a.x_out + blk * 8) = xw;
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // the scale row's loads go out before the reductions
+  u32x4 sr[NB <= 8 ? NB : 1];
+  if constexpr (NB <= 8) {
+#pragma unroll
+    for (int j = 0; j < NB; j++) sr[j] = *reinterpret_cast<const u32x4*>(prm + D + (cb0 + 64 * j) * 8);
+  }
+  auto row_sum = [&](int i, float p) {
+    p = sum_rib(p);
+    if (lane < kLsRows) red[i][wave][lane] = p;
+    __syncthreads();
+    float t = 0.f;
+#pragma unroll
+    for (int w = 0; w < kLsThreads / 64; w++) t += red[i][w][rib];
+    return t;
+  };
+  float mean = 0.f;
+  if (a.norm == RL_NORM_LAYER) mean = row_sum(0, s) / (float)D;
+  float ss = 0.f;
+#pragma unroll
+  for (int j = 0; j < NB; j++) {
+    float xf[8];
+    unpack8(v[j], xf);
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const float d = xf[e] - mean;
+      ss = fmaf(d, d, ss);
+    }
+  }
+  const float rstd = __builtin_amdgcn_rsqf(row_sum(1, ss) / (float)D + 1e-6f);
+
+  // y -> bfp16; the 8 rows' blocks of column block cb are 72 consecutive bytes of the A layout, staged at 72 cb
+#pragma unroll
+  for (int j = 0; j < NB; j++) {
+    const int cb = cb0 + 64 * j;
+    float sf[8], xf[8];
+    if constexpr (NB <= 8)
+      unpack8(sr[j], sf);
+    else
+      unpack8(*reinterpret_cast<const u32x4*>(prm + D + cb * 8), sf);
+    unpack8(v[j], xf);
+    uint32_t u[8];
+    int32_t q[8];
+    u32x4 bw;
+#pragma unroll
+    for (int e = 0; e < 8; e++) u[e] = __float_as_uint((xf[e] - mean) * rstd * sf[e]);
+    const uint32_t E = encode_block(u, q, bw);
+    uint8_t* p = stage + (cb * 8 + rib) * kBlockBytes;
+    p[0] = (uint8_t)E;
+#pragma unroll
+    for (int e = 0; e < 8; e++) p[1 + e] = (uint8_t)(int8_t)q[e];
+  }
+  __syncthreads();
+  // A tile (mt, kt): 8 bands x 8 column blocks x 144 bytes, of which this workgroup's half is 72
+  const int64_t KT = D >> 6;
+  uint8_t* dst = a.a_packed + ((r0 >> 7) * KT * 8 + ((r0 >> 4) & 7)) * 1152 + ((r0 >> 3) & 1) * 72;
+  for (int c = tid; c < (D >> 3) * 9; c += kLsThreads) {
+    const int cb = c / 9, w = c - cb * 9;
+    *reinterpret_cast<uint2*>(dst + (cb >> 3) * (8 * 1152) + (cb & 7) * 144 + 8 * w) =
+        *reinterpret_cast<const uint2*>(stage + 8 * c);
+  }
+}
+
+template <int NB>
+static int launch_stream(const LnStreamArgs& a, int br, int64_t M, hipStream_t st) {
+  const dim3 grid((unsigned)(M / kLsRows)), block(kLsThreads);
+  const int lds = a.D * kBlockBytes;  // 8 rows x D / 8 blocks
+  auto go = [&](auto kernel) {
+    if (lds > 48 * 1024) {
+      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+      if (e != hipSuccess) return fail(RL_ERR_DEVICE, "hipFuncSetAttribute: %s", hipGetErrorString(e));
+    }
+    hipLaunchKernelGGL(kernel, grid, block, (unsigned)lds, st, a);
+    return launch_status("rl_ln_modulate_stream");
+  };
+  if (br == 0) return go(ln_stream_kernel<NB, 0>);
+  return br == 1 ? go(ln_stream_kernel<NB, 1>) : go(ln_stream_kernel<NB, 2>);
+}
+
 }  // namespace rl
 
 extern "C" int rl_ln_modulate(const uint16_t* x, int64_t ldx, const void* branch, int32_t br_fmt, int64_t ld_br,
@@ -332,4 +517,36 @@ extern "C" int rl_ln_modulate(const uint16_t* x, int64_t ldx, const void* branch
   a.rows_wg = (a_packed && a_order == RL_ORDER_A_LAYOUT) ? 16 : 4;
   const int nb = (int)((D / 8 + 63) / 64);
   return launch_upto<1>(nb, a, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int rl_ln_modulate_stream(const uint16_t* x, const void* branch, int32_t br_fmt, const uint16_t* params,
+                                     int64_t split_row, int32_t norm, uint16_t* x_out, uint8_t* a_packed, int64_t M,
+                                     int64_t D, void* stream) {
+  using namespace rl;
+  int s = rl_validate_ln(D, br_fmt, D, norm, D, RL_ORDER_A_LAYOUT, D, split_row, M, D);
+  if (s) return s;
+  if (M % 512 || D % 1024)
+    return fail(RL_ERR_SHAPE, "M %lld D %lld: the C-stream order needs M %% 512 == 0 and D %% 1024 == 0", (long long)M,
+                (long long)D);
+  if (!x || !params || !x_out || !a_packed) return fail(RL_ERR_NULL, "x, params, x_out or a_packed is NULL");
+  if (((uintptr_t)x | (uintptr_t)params | (uintptr_t)x_out | (uintptr_t)a_packed) % 16)
+    return fail(RL_ERR_ALIGN, "x, params and the outputs must be 16-byte aligned");
+  if (branch && (uintptr_t)branch % (br_fmt == RL_BRANCH_BF16 ? 16 : 4))
+    return fail(RL_ERR_ALIGN, "branch must be 16-byte (bf16) or 4-byte (packed) aligned");
+  if ((s = check_device())) return s;
+  LnStreamArgs a;
+  a.x = x; a.br = branch; a.params = params; a.split_row = split_row; a.norm = norm;
+  a.x_out = x_out; a.a_packed = a_packed; a.D = (int32_t)D;
+  const int br = !branch ? 0 : br_fmt == RL_BRANCH_BF16 ? 1 : 2;
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  switch (D / 1024) {
+    case 1: return launch_stream<2>(a, br, M, st);
+    case 2: return launch_stream<4>(a, br, M, st);
+    case 3: return launch_stream<6>(a, br, M, st);
+    case 4: return launch_stream<8>(a, br, M, st);
+    case 5: return launch_stream<10>(a, br, M, st);
+    case 6: return launch_stream<12>(a, br, M, st);
+    case 7: return launch_stream<14>(a, br, M, st);
+    default: return launch_stream<16>(a, br, M, st);
+  }
 }

@@ -332,6 +332,27 @@ def ln_modulate(x, params, branch=None, split_row=0, norm="layer", x_out=None, p
     return x_out, a_p, a_d
 
 
+def overlaps(a, b):
+    """Whether two contiguous device tensors share memory."""
+    return a.data_ptr() < b.data_ptr() + b.numel() * b.element_size() and \
+        b.data_ptr() < a.data_ptr() + a.numel() * a.element_size()
+
+
+def stream_buffer(t, dtype, numel, align=16):
+    """Whether t can be read or written by a stream kernel in place: a contiguous device tensor of `dtype` with exactly
+    `numel` elements and an aligned address."""
+    return t.device.type == "cuda" and t.dtype == dtype and t.is_contiguous() and t.numel() == numel and \
+        t.data_ptr() % align == 0
+
+
+def ln_modulate_stream(x, params, branch, x_out, a_out, M, D, split_row=0, norm="layer"):
+    """ln_modulate on the C-stream element order: x, x_out flat bf16, branch None, flat bf16 or a uint8 bfp16 stream in
+    that order, a_out the uint8 buffer that receives A in the A layout. See rl_ln_modulate_stream in include/rlbfp.h."""
+    fmt = L.RL_BRANCH_PACKED if branch is not None and branch.dtype == torch.uint8 else L.RL_BRANCH_BF16
+    L.check(L.lib().rl_ln_modulate_stream(_ptr(x), _ptr(branch), fmt, _ptr(params), split_row, _NORMS[norm],
+                                          _ptr(x_out), _ptr(a_out), M, D, _stream(x)))
+
+
 # ---------------------------------------------------------------------------------------------------------------
 # QKV post -> attention Q / K / V
 # ---------------------------------------------------------------------------------------------------------------

@@ -50,12 +50,38 @@ def rows_param(v, M, S):
     return out
 
 
+def _stream_form(X, BR, P, XO, AO, M, d):
+    """Whether the buffers are the artifact's own: whole, contiguous C-order streams on one device with a packed A
+    that rl_ln_modulate_stream reads and writes in place. Outputs over inputs (other than XO = X) take the general
+    form, which writes them only after everything has been read."""
+    n = M * d
+    if X.dim() != 1 or XO.dim() != 1 or M % 512 or d % 1024 or not 1024 <= d <= 8192:
+        return False
+    if not (ops.stream_buffer(X, torch.bfloat16, n) and ops.stream_buffer(XO, torch.bfloat16, n) and
+            ops.stream_buffer(AO, torch.uint8, n // 8 * 9) and ops.stream_buffer(P, torch.bfloat16, 4 * d)):
+        return False
+    ins = [P]
+    if BR is not None:
+        if not (ops.stream_buffer(BR, torch.uint8, n // 8 * 9, 4) or
+                BR.dim() == 1 and ops.stream_buffer(BR, torch.bfloat16, n)):
+            return False
+        ins.append(BR)
+    if any(t.device != X.device for t in ins + [XO, AO]):
+        return False
+    if X.data_ptr() != XO.data_ptr():
+        ins.append(X)
+    return not (any(ops.overlaps(o, t) for o in (XO, AO) for t in ins) or ops.overlaps(AO, XO))
+
+
 def ln_fused(art, X, BR, P, XO, AO):
     """x' = bf16(x + g * BR), A = LayerNorm(x') * sc (or RMSNorm) as bfp16; see the module docstring for the forms."""
     S, norm = art_params(art)
     d = P.numel() // 4
     stream = X.dim() == 1
     M = X.numel() // d
+    if stream and _stream_form(X, BR, P, XO, AO, M, d):
+        ops.ln_modulate_stream(X, P, BR, XO, AO, M, d, split_row=S * 128, norm=norm)
+        return
     x = layouts.c_unlayout_atb_values(X, M, d) if stream else X
     if BR is None:
         br = None

@@ -247,3 +247,13 @@ def test_validate_qkv_post_gqa(args, code):
 def test_qkv_post_gqa_null_pointers_rejected_before_any_gpu_call():
     assert L.lib().rl_qkv_post_gqa(None, 6144, 64, 32, 8, None, None, None, None, None, None, None, None, None,
                                    None) == L.RL_ERR_NULL
+
+
+def test_ln_stream_rejects_before_any_gpu_call():
+    f = L.lib().rl_ln_modulate_stream
+    assert f(16, None, 0, 16, 0, 0, 16, 16, 500, 1024, None) == L.RL_ERR_SHAPE   # M % 512
+    assert f(16, None, 0, 16, 0, 0, 16, 16, 512, 1088, None) == L.RL_ERR_SHAPE   # D % 1024
+    assert f(16, None, 0, 16, 0, 0, 16, 16, 512, 9216, None) == L.RL_ERR_SHAPE   # D > 8192
+    assert f(16, None, 2, 16, 0, 0, 16, 16, 512, 1024, None) == L.RL_ERR_ARG
+    assert f(16, None, 0, 16, 0, 0, None, 16, 512, 1024, None) == L.RL_ERR_NULL
+    assert f(16, None, 0, 16, 0, 0, 16, 8, 512, 1024, None) == L.RL_ERR_ALIGN
