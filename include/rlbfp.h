@@ -282,6 +282,23 @@ int rl_attention_ws(const uint16_t *q, const uint16_t *k, const uint16_t *vt, in
  * shape is invalid). Without a usable device the plan assumes 256 compute units. */
 int64_t rl_attention_workspace_bytes(int32_t heads, int64_t nq, int64_t nk);
 
+/* The attention artifacts' own formats around the same kernel (redline/run_attn.py:27-34, :67-82).
+ * rl_attn_tiles decodes packed 64-token tiles (rl_qkv_post's q_tiles / kv_tiles) into rl_attention's operands: tiles
+ * q_first .. q_first + q_count - 1 of the q_all tiles per head in q_tiles -> q (hq, nq, 128), rows past them zero; then
+ * count0 tiles of kv0 and count1 of kv1 (count1 = 0: one buffer) per K / V head, in that order -> k (hkv, nk, 128) and
+ * vt (hkv, 128, nk), nk = 64 (count0 + count1). Exact. Tiles 4-byte, outputs 16-byte aligned; nq % 64 == 0.
+ * rl_attention_packed is rl_attention_ws with kv_heads K / V heads (query head h reads head h / (heads / kv_heads))
+ * whose O, quantized to bfp16 blocks of 8 dims, goes out packed in RL_ORDER_A_LAYOUT of an (o_rows, o_cols) matrix:
+ * rows 0 .. rows - 1, columns (h0 + h) * 128 ..; the stream's other blocks are left as they are. o_rows % 128 == 0,
+ * o_cols % 64 == 0, rows % 16 == 0, rows <= nq and o_rows. Workspace as for rl_attention_ws (same byte count). */
+int rl_attn_tiles(const uint8_t *q_tiles, int32_t hq, int64_t q_all, int64_t q_first, int64_t q_count, int64_t nq,
+                  uint16_t *q, const uint8_t *kv0, int64_t all0, int64_t first0, int64_t count0, const uint8_t *kv1,
+                  int64_t all1, int64_t first1, int64_t count1, int32_t hkv, uint16_t *k, uint16_t *vt, void *stream);
+int rl_attention_packed(const uint16_t *q, const uint16_t *k, const uint16_t *vt, int32_t heads, int32_t kv_heads,
+                        int64_t nq, int64_t nk, int64_t nkv, const int32_t *lim, uint8_t *o, int64_t o_rows,
+                        int64_t o_cols, int32_t h0, int64_t rows, void *workspace, int64_t workspace_bytes,
+                        void *stream);
+
 /* ---- host-only helpers (no GPU needed) ---------------------------------------------------------------------------- */
 /* Shape/argument checks the entry points run before launching, callable on a machine without a GPU. */
 int rl_validate_ln(int64_t ldx, int32_t br_fmt, int64_t ld_br, int32_t norm, int64_t ld_xo, int32_t a_order,

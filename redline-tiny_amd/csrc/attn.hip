@@ -50,6 +50,12 @@ struct AttnArgs {
   int32_t nkv;
   const int32_t* lim;
   int32_t quantize;
+  // packed output (attn_kernel<W, true>): O as bfp16 in the A layout of a matrix of okt 64-column tiles, rows below
+  // orows; o and ldo are not used then
+  uint8_t* o9;
+  int32_t okt;
+  int32_t orows;
+  int32_t gq;  // query heads per K / V head
   // work split (see attn_plan): tasks below nfull run whole; the rest in ranges of `per` key blocks, a task cut by a
   // range boundary leaving one partial per range in ws (mp slots per tail task)
   int32_t ntask;
@@ -58,6 +64,39 @@ struct AttnArgs {
   int32_t mp;
   float* ws;
 };
+
+// (head, query block) of a task. Without per-query limits a head's query blocks are adjacent (its K and V^T stay in
+// the L2 of the XCDs that work on it). With limits, tasks clip their key range to the largest limit of their queries,
+// so under a causal mask the last query blocks take longest: those of all heads come first.
+__device__ __forceinline__ void task_pos(int task, int heads, int nqb, bool lim, int& h, int& qb) {
+  if (lim) {
+    qb = nqb - 1 - task / heads;
+    h = task % heads;
+  } else {
+    h = task / nqb;
+    qb = task - h * nqb;
+  }
+}
+
+// The q byte of one element of a block with exponent E, as encode_block gives it
+__device__ __forceinline__ uint8_t encode_with_exp(uint32_t u, uint32_t E) {
+  if (E >= kFastEMin && E <= kFastEMax) return (uint8_t)__float_as_uint(encode_fast(__uint_as_float(u), block_scales(E)));
+  return (uint8_t)encode_elem(u, E);
+}
+
+// Byte offset of the 16-row band of row r (r % 16 == 0) in tile column kt of an A-layout stream with okt tile columns:
+// 128 blocks, 1152 consecutive bytes; the band's next tile column is 8 * 1152 bytes on
+__device__ __forceinline__ int64_t band_offset(int r, int kt, int okt) {
+  return (((int64_t)(r >> 7) * okt + kt) * 8 + ((r >> 4) & 7)) * 1152;
+}
+
+// The lane index, computed where it stands: addresses derived from it are not hoisted out of the key loop, where they
+// would hold registers that the loop needs
+__device__ __forceinline__ int lane_here() {
+  int zero = 0;
+  asm volatile("" : "+s"(zero));
+  return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
+}
 
 __device__ __forceinline__ f32x4 mfma16(bf16x8 a, bf16x8 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -98,7 +137,9 @@ constexpr int part_floats(int q) { return q * kAtHD + 2 * q; }
 // W waves per workgroup (4 or 8), 32 queries each; two 4-wave or one 8-wave workgroup per CU (256 VGPRs per wave,
 // 64 KB of LDS per workgroup). The 8 waves of the larger workgroup meet at every key block's barrier, so they
 // progress together, and each staged key block serves 256 queries.
-template <int W>
+// PK: O goes out as bfp16 blocks in the A layout (staged in the K / V buffers, 16-byte stores) instead of bf16 rows.
+// LIM: per-query key limits are given (their registers and the clipping are compiled out otherwise).
+template <int W, bool PK, bool LIM>
 __global__ __launch_bounds__(W * 64, 8 / W) void attn_kernel(AttnArgs a) {
   constexpr int kAtThreads = W * 64, kAtQ = W * kAtQW, kAtPart = part_floats(kAtQ);
   constexpr int NI = 16 / W;  // 16-byte staging chunks per thread per K (and per V^T) block
@@ -122,11 +163,13 @@ __global__ __launch_bounds__(W * 64, 8 / W) void attn_kernel(AttnArgs a) {
     const int task = f / nblk, kb0 = f - task * nblk, kb1 = min(nblk, f1 - task * nblk);
     if (f > f0) __syncthreads();  // a second segment reuses the LDS buffers
     f = task * nblk + kb1;
-    const int h = task / nqb, qb = task - h * nqb;
+    int h, qb;
+    task_pos(task, a.heads, nqb, LIM, h, qb);
     const int q0 = qb * kAtQ + wave * kAtQW;
+    const int hk = h / a.gq;
     const uint16_t* Qh = a.q + (int64_t)h * a.nq * kAtHD;
-    const uint16_t* Kh = a.k + (int64_t)h * a.nk * kAtHD;
-    const uint16_t* Vh = a.vt + (int64_t)h * kAtHD * a.nk;
+    const uint16_t* Kh = a.k + (int64_t)hk * a.nk * kAtHD;
+    const uint16_t* Vh = a.vt + (int64_t)hk * kAtHD * a.nk;
 
     // Q^T as the B operand: set s, 32-dim step st: Q[q0 + 16 s + l16][32 st + 8 lg .. + 7]
     bf16x8 qB[2][4];
@@ -135,9 +178,21 @@ __global__ __launch_bounds__(W * 64, 8 / W) void attn_kernel(AttnArgs a) {
 #pragma unroll
       for (int st = 0; st < 4; st++)
         qB[s][st] = *reinterpret_cast<const bf16x8*>(Qh + (int64_t)(q0 + 16 * s + l16) * kAtHD + 32 * st + 8 * lg);
-    int lim[2];
+    // keys below `vis` are visible to all of the wave's queries, keys from `end` on to none of the workgroup's: key
+    // blocks past `end` are not read, blocks below `vis` not masked
+    int vis = a.nkv, end = a.nkv;
+    if constexpr (LIM) {
+      int lo = min(a.lim[q0 + l16], a.lim[q0 + 16 + l16]), hi = -1;
 #pragma unroll
-    for (int s = 0; s < 2; s++) lim[s] = a.lim ? a.lim[q0 + 16 * s + l16] : 0x7FFFFFFF;
+      for (int i = 0; i < kAtQ / 64; i++) hi = max(hi, a.lim[qb * kAtQ + 64 * i + lane]);
+#pragma unroll
+      for (int x = 32; x >= 1; x >>= 1) {
+        lo = min(lo, __shfl_xor(lo, x));
+        hi = max(hi, __shfl_xor(hi, x));
+      }
+      vis = min(vis, __builtin_amdgcn_readfirstlane(max(lo, -1)) + 1);
+      end = min(end, __builtin_amdgcn_readfirstlane(min(hi, a.nkv)) + 1);
+    }
 
     f32x4 O[2][8];
 #pragma unroll
@@ -224,16 +279,17 @@ __global__ __launch_bounds__(W * 64, 8 / W) void attn_kernel(AttnArgs a) {
     // (after its P V products of the previous block) when the running max was rebased, rebased[s] whether any lane of
     // the set did. The four lanes l16, l16 + 16, + 32, + 48 hold a query's 64 keys.
     auto softmax = [&](int b, u32x4 (&Pb)[2][2], float (&alpha)[2], bool (&rebased)[2]) {
-      const bool full = (b + 1) * kAtKB <= a.nkv && !a.lim;
+      const bool full = (b + 1) * kAtKB <= vis;
 #pragma unroll
       for (int s = 0; s < 2; s++) {
         if (!full) {
+          const int lim = LIM ? a.lim[q0 + 16 * s + (lane_here() & 15)] : 0x7FFFFFFF;
 #pragma unroll
           for (int g = 0; g < 4; g++)
 #pragma unroll
             for (int i = 0; i < 4; i++) {
               const int key = b * kAtKB + 16 * g + 4 * lg + i;
-              if (key >= a.nkv || key > lim[s]) S[s][g][i] = -INFINITY;
+              if (key >= a.nkv || key > lim) S[s][g][i] = -INFINITY;
             }
         }
         float mx = S[s][0][0];
@@ -297,7 +353,9 @@ __global__ __launch_bounds__(W * 64, 8 / W) void attn_kernel(AttnArgs a) {
       }
     };
 
-    const int nb = kb1 - kb0;  // key blocks kb0 .. kb1 - 1; segment-relative index r = block - kb0
+    // key blocks kb0 .. kb0 + nb - 1 (at least one, which a segment past every limit masks whole); segment-relative
+    // index r = block - kb0
+    const int nb = max(1, min(kb1, (end + kAtKB - 1) / kAtKB) - kb0);
     load_k(kb0);
     load_v(kb0);
     store_k(0);
@@ -351,7 +409,8 @@ __global__ __launch_bounds__(W * 64, 8 / W) void attn_kernel(AttnArgs a) {
       float* part = a.ws + ((int64_t)u * a.mp + (ti - u * nblk / a.per)) * kAtPart;
 #pragma unroll
       for (int s = 0; s < 2; s++) {
-        const int ql = wave * kAtQW + 16 * s + l16;
+        const int ln = lane_here(), lg = ln >> 4;
+        const int ql = wave * kAtQW + 16 * s + (ln & 15);
         const float l = sum4(lsum[s]);
 #pragma unroll
         for (int dg = 0; dg < 8; dg++) *reinterpret_cast<f32x4*>(part + ql * kAtHD + 16 * dg + 4 * lg) = O[s][dg];
@@ -364,11 +423,49 @@ __global__ __launch_bounds__(W * 64, 8 / W) void attn_kernel(AttnArgs a) {
     }
 
     // O = O^T / l: lane holds dims 16 dg + 4 lg + i of query q0 + 16 s + l16
+    if constexpr (PK) {
+      // the wave's two 16-query bands, each 16 column blocks x 16 rows x 9 bytes (one band of two A-layout tile
+      // columns), staged in the wave's own part of the K / V buffers
+      __syncthreads();  // the last block's K and V reads of every wave are done
+      const int ln = lane_here(), lr = ln & 15, lq = ln >> 4;
+      uint8_t* st = lds + wave * (2 * 2304);
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        const float l = sum4(lsum[s]);
+        const float inv = l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+        for (int dg = 0; dg < 8; dg++) {
+          uint32_t u[4], E = 0;
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            u[i] = __float_as_uint(O[s][dg][i] * inv);
+            E = max(E, (u[i] >> 23) & 0xFFu);
+          }
+          const auto r = __builtin_amdgcn_permlane16_swap(E, E, false, false);
+          E = max((uint32_t)r[0], (uint32_t)r[1]);
+          uint8_t* b = st + s * 2304 + ((2 * dg + (lq >> 1)) * 16 + lr) * kBlockBytes;
+          if (!(lq & 1)) b[0] = (uint8_t)E;
+#pragma unroll
+          for (int i = 0; i < 4; i++) b[1 + 4 * (lq & 1) + i] = encode_with_exp(u[i], E);
+        }
+      }
+      __syncthreads();
+#pragma unroll
+      for (int s = 0; s < 2; s++) {
+        if (q0 + 16 * s >= a.orows) break;
+        uint8_t* dst = a.o9 + band_offset(q0 + 16 * s, 2 * (a.h0 + h), a.okt);
+        for (int c = ln; c < 144; c += 64)
+          *reinterpret_cast<u32x4*>(dst + (c >= 72 ? 7 * 1152 : 0) + 16 * c) =
+              *reinterpret_cast<const u32x4*>(st + s * 2304 + 16 * c);
+      }
+      continue;
+    }
 #pragma unroll
     for (int s = 0; s < 2; s++) {
       const float l = sum4(lsum[s]);
       const float inv = l > 0.f ? 1.f / l : 0.f;
-      uint16_t* orow = a.o + (int64_t)(q0 + 16 * s + l16) * a.ldo + (int64_t)(a.h0 + h) * kAtHD;
+      const int ln = lane_here(), lg = ln >> 4;
+      uint16_t* orow = a.o + (int64_t)(q0 + 16 * s + (ln & 15)) * a.ldo + (int64_t)(a.h0 + h) * kAtHD;
 #pragma unroll
       for (int dg = 0; dg < 8; dg++) {
         uint32_t u[4], b[4];
@@ -410,6 +507,11 @@ struct CombineArgs {
   int32_t mp;
   int32_t quantize;
   int32_t qt;  // queries per task (128 or 256)
+  int32_t heads;
+  int32_t lim;  // task order (task_pos)
+  uint8_t* o9;  // packed output as in AttnArgs, or NULL
+  int32_t okt;
+  int32_t orows;
 };
 
 constexpr int kCbQ = 16;  // queries per combine workgroup
@@ -421,7 +523,8 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(CombineArgs c) {
   const int p0 = u * nblk / c.per, p1 = (u * nblk + nblk - 1) / c.per;
   if (p0 == p1) return;  // the task lay inside one range and was written whole
   const int np = p1 - p0 + 1;
-  const int h = task / nqb, qb = task - h * nqb;
+  int h, qb;
+  task_pos(task, c.heads, nqb, c.lim != 0, h, qb);
   const int ql = qs * kCbQ + (threadIdx.x >> 4), d8 = threadIdx.x & 15;
   const float* base = c.ws + (int64_t)u * c.mp * kAtPart;
   float mx = -INFINITY;
@@ -461,6 +564,22 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(CombineArgs c) {
   uint32_t uu[8], b[8];
 #pragma unroll
   for (int i = 0; i < 8; i++) uu[i] = __float_as_uint(acc[i] * inv);
+  if (c.o9) {
+    // 16 queries x 16 column blocks: one band of two A-layout tile columns
+    __shared__ __attribute__((aligned(16))) uint8_t st[2304];
+    int32_t q[8];
+    u32x4 bw;
+    uint8_t* p = st + (d8 * 16 + (threadIdx.x >> 4)) * kBlockBytes;
+    p[0] = (uint8_t)encode_block(uu, q, bw);
+#pragma unroll
+    for (int i = 0; i < 8; i++) p[1 + i] = (uint8_t)q[i];
+    __syncthreads();
+    const int row = qb * kAtQ + qs * kCbQ, w = threadIdx.x;
+    if (row < c.orows && w < 144)
+      *reinterpret_cast<u32x4*>(c.o9 + band_offset(row, 2 * (c.h0 + h), c.okt) + (w >= 72 ? 7 * 1152 : 0) + 16 * w) =
+          *reinterpret_cast<const u32x4*>(st + 16 * w);
+    return;
+  }
   uint16_t* orow = c.o + (int64_t)(qb * kAtQ + ql) * c.ldo + (int64_t)(c.h0 + h) * kAtHD + 8 * d8;
   if (c.quantize) {
     uint32_t E = 0;
@@ -522,6 +641,37 @@ extern "C" int64_t rl_attention_workspace_bytes(int32_t heads, int64_t nq, int64
   return attn_plan(heads, nq, nk, device_cus()).ws_floats * 4;
 }
 
+namespace rl {
+// The launches of one attention call whose arguments have been checked; `a` carries everything but the work split.
+static int attn_launch(AttnArgs a, void* workspace, int64_t workspace_bytes, hipStream_t st) {
+  int s;
+  AttnPlan plan = attn_plan(a.heads, a.nq, a.nk, device_cus());
+  if (!workspace) plan = attn_plan(a.heads, a.nq, a.nk, 0);  // no workspace: every task whole
+  if (plan.ws_floats * 4 > workspace_bytes && plan.ws_floats > 0)
+    return fail(RL_ERR_WORKSPACE, "workspace %lld bytes, this shape needs %lld (rl_attention_workspace_bytes)",
+                (long long)workspace_bytes, (long long)(plan.ws_floats * 4));
+  a.ntask = plan.ntask; a.nfull = plan.nfull; a.per = plan.per; a.mp = plan.mp;
+  a.ws = static_cast<float*>(workspace);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)plan.nwg), dim3(plan.w * 64), 0, st, a);
+  };
+  auto pick = [&]<int W, bool PK>() { a.lim ? go(attn_kernel<W, PK, true>) : go(attn_kernel<W, PK, false>); };
+  if (plan.w == 8)
+    a.o9 ? pick.template operator()<8, true>() : pick.template operator()<8, false>();
+  else
+    a.o9 ? pick.template operator()<4, true>() : pick.template operator()<4, false>();
+  if ((s = launch_status("rl_attention"))) return s;
+  if (plan.nfull == plan.ntask) return RL_OK;
+  CombineArgs c;
+  c.ws = a.ws; c.o = a.o; c.ldo = a.ldo; c.h0 = a.h0; c.nq = a.nq; c.nk = a.nk; c.nfull = plan.nfull;
+  c.per = plan.per; c.mp = plan.mp; c.quantize = a.quantize; c.qt = plan.w * kAtQW;
+  c.heads = a.heads; c.lim = a.lim != nullptr; c.o9 = a.o9; c.okt = a.okt; c.orows = a.orows;
+  hipLaunchKernelGGL(attn_combine_kernel, dim3((unsigned)((plan.ntask - plan.nfull) * (c.qt / kCbQ))), dim3(256),
+                     0, st, c);
+  return launch_status("rl_attention (combine)");
+}
+}  // namespace rl
+
 extern "C" int rl_attention_ws(const uint16_t* q, const uint16_t* k, const uint16_t* vt, int32_t heads, int64_t nq,
                                int64_t nk, int64_t nkv, const int32_t* lim, uint16_t* o, int64_t ldo, int32_t h0,
                                int32_t quantize_out, void* workspace, int64_t workspace_bytes, void* stream) {
@@ -532,30 +682,36 @@ extern "C" int rl_attention_ws(const uint16_t* q, const uint16_t* k, const uint1
   if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)vt | (uintptr_t)o | (uintptr_t)workspace) % 16 || (uintptr_t)lim % 4)
     return fail(RL_ERR_ALIGN, "q, k, vt, o and the workspace must be 16-byte aligned, lim 4-byte aligned");
   if ((s = check_device())) return s;
-  AttnPlan plan = attn_plan(heads, nq, nk, device_cus());
-  if (!workspace) plan = attn_plan(heads, nq, nk, 0);  // no workspace: every task whole
-  if (plan.ws_floats * 4 > workspace_bytes && plan.ws_floats > 0)
-    return fail(RL_ERR_WORKSPACE, "workspace %lld bytes, this shape needs %lld (rl_attention_workspace_bytes)",
-                (long long)workspace_bytes, (long long)(plan.ws_floats * 4));
-  AttnArgs a;
+  AttnArgs a = {};
   a.q = q; a.k = k; a.vt = vt; a.o = o; a.ldo = ldo; a.h0 = h0;
   a.heads = heads; a.nq = (int32_t)nq; a.nk = (int32_t)nk; a.nkv = (int32_t)nkv; a.lim = lim;
   a.quantize = quantize_out ? 1 : 0;
-  a.ntask = plan.ntask; a.nfull = plan.nfull; a.per = plan.per; a.mp = plan.mp;
-  a.ws = static_cast<float*>(workspace);
-  const hipStream_t st = static_cast<hipStream_t>(stream);
-  if (plan.w == 8)
-    hipLaunchKernelGGL(attn_kernel<8>, dim3((unsigned)plan.nwg), dim3(512), 0, st, a);
-  else
-    hipLaunchKernelGGL(attn_kernel<4>, dim3((unsigned)plan.nwg), dim3(256), 0, st, a);
-  if ((s = launch_status("rl_attention"))) return s;
-  if (plan.nfull == plan.ntask) return RL_OK;
-  CombineArgs c;
-  c.ws = a.ws; c.o = o; c.ldo = ldo; c.h0 = h0; c.nq = a.nq; c.nk = a.nk; c.nfull = plan.nfull; c.per = plan.per;
-  c.mp = plan.mp; c.quantize = a.quantize; c.qt = plan.w * kAtQW;
-  hipLaunchKernelGGL(attn_combine_kernel, dim3((unsigned)((plan.ntask - plan.nfull) * (c.qt / kCbQ))), dim3(256),
-                     0, st, c);
-  return launch_status("rl_attention (combine)");
+  a.gq = 1;
+  return attn_launch(a, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
+}
+
+extern "C" int rl_attention_packed(const uint16_t* q, const uint16_t* k, const uint16_t* vt, int32_t heads,
+                                   int32_t kv_heads, int64_t nq, int64_t nk, int64_t nkv, const int32_t* lim,
+                                   uint8_t* o, int64_t o_rows, int64_t o_cols, int32_t h0, int64_t rows,
+                                   void* workspace, int64_t workspace_bytes, void* stream) {
+  using namespace rl;
+  int s = rl_validate_attention(heads, nq, nk, nkv, o_cols, h0);
+  if (s) return s;
+  if (kv_heads < 1 || heads % kv_heads) return fail(RL_ERR_SHAPE, "%d heads over %d K / V heads", heads, kv_heads);
+  if (o_rows < 128 || o_rows % 128 || o_rows > (1 << 30) || o_cols % 64 || o_cols > (1 << 30) || rows < 16 ||
+      rows % 16 || rows > nq || rows > o_rows)
+    return fail(RL_ERR_SHAPE, "O %lld x %lld, %lld rows: need o_rows %% 128 == 0, o_cols %% 64 == 0, rows %% 16 == 0 "
+                "and rows <= nq, o_rows", (long long)o_rows, (long long)o_cols, (long long)rows);
+  if (!q || !k || !vt || !o) return fail(RL_ERR_NULL, "q, k, vt or o is NULL");
+  if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)vt | (uintptr_t)o | (uintptr_t)workspace) % 16 || (uintptr_t)lim % 4)
+    return fail(RL_ERR_ALIGN, "q, k, vt, o and the workspace must be 16-byte aligned, lim 4-byte aligned");
+  if ((s = check_device())) return s;
+  AttnArgs a = {};
+  a.q = q; a.k = k; a.vt = vt; a.h0 = h0;
+  a.heads = heads; a.nq = (int32_t)nq; a.nk = (int32_t)nk; a.nkv = (int32_t)nkv; a.lim = lim;
+  a.gq = heads / kv_heads;
+  a.o9 = o; a.okt = (int32_t)(o_cols / 64); a.orows = (int32_t)rows;
+  return attn_launch(a, workspace, workspace_bytes, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int rl_attention(const uint16_t* q, const uint16_t* k, const uint16_t* vt, int32_t heads, int64_t nq,

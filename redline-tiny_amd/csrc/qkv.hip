@@ -173,6 +173,75 @@ __global__ __launch_bounds__(kQkvThreads) void qkv_post_kernel(QkvArgs a) {
     *reinterpret_cast<u32x4*>(dst + 16 * c) = *reinterpret_cast<const u32x4*>(&stage[16 * c]);
 }
 
+// ---- attention tiles -> the attention kernel's operands --------------------------------------------------------------
+//
+// One workgroup decodes one 9216-byte tile: Q and K tiles to 64 rows of 256 bytes (head major), V tiles to 128 rows of
+// V^T, 128 bytes each; query tiles past the source range are zeros. Thread t decodes blocks 4 t .. 4 t + 3, a 36-byte
+// dword-aligned run (two 16-byte loads and one 4-byte load) holding rows r .. r + 3 (V: dims) of one 8-value block
+// column, so each store instruction of a wave fills whole 256-byte (V: 128-byte) rows. HBM-bound: 9/8 bytes read and 2
+// written per value; it replaces index-tensor gathers, float32 copies and concatenations of every operand (32 heads, 4096
+// queries, 8256 keys, with the packed O below: the whole attention step 4960 -> 1155 us). Decoding inside the attention kernel instead would cost every workgroup of a head the same ~100
+// VALU instructions per wave and key block, beside 112 of the softmax.
+struct TilesArgs {
+  const uint8_t* q_tiles;
+  int32_t hq, q_all, q_t0, q_n, q_out;  // heads, tiles per head in the source, first tile, tiles there, tiles written
+  uint16_t* q;
+  const uint8_t* kv[2];  // [head][tile][K | V]; the second may be absent (n = 0)
+  int32_t hkv, kv_all[2], kv_t0[2], kv_n[2];
+  uint16_t* k;
+  uint16_t* vt;
+};
+
+__global__ __launch_bounds__(kQkvThreads) void attn_tiles_kernel(TilesArgs a) {
+  typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
+  const int tid = threadIdx.x;
+  const int nkt = a.kv_n[0] + a.kv_n[1];
+  const int64_t nk = (int64_t)nkt * kTileTokens;
+  int j = blockIdx.x;
+  const uint8_t* src;
+  uint16_t* dst;
+  int64_t ld;
+  int row, col;
+  bool zero = false;
+  const int nq = a.hq * a.q_out;
+  if (j < nq || ((j - nq) & 1) == 0) {
+    // Q and K: blocks (16-token band, 8-dim block, 8-token half, token)
+    row = (tid >> 6) * 16 + (tid & 3) * 4;
+    col = (tid >> 2) & 15;
+    ld = kHeadDim;
+  } else {
+    // V: blocks (16-dim band, 8-token block, 8-dim half, dim)
+    row = (tid >> 5) * 16 + (tid & 3) * 4;
+    col = (tid >> 2) & 7;
+    ld = nk;
+  }
+  if (j < nq) {
+    const int h = j / a.q_out, t = j - h * a.q_out;
+    zero = t >= a.q_n;
+    src = a.q_tiles + ((int64_t)h * a.q_all + a.q_t0 + t) * kTile9;
+    dst = a.q + (int64_t)j * kTileTokens * kHeadDim;
+  } else {
+    j -= nq;
+    const int v = j & 1, h = (j >> 1) / nkt, t = (j >> 1) - h * nkt;
+    const int b = t >= a.kv_n[0];
+    src = a.kv[b] + (((int64_t)h * a.kv_all[b] + a.kv_t0[b] + (b ? t - a.kv_n[0] : t)) * 2 + v) * kTile9;
+    dst = v ? a.vt + (int64_t)h * kHeadDim * nk + t * kTileTokens
+            : a.k + ((int64_t)h * nk + t * kTileTokens) * kHeadDim;
+  }
+  u32x4 o[4] = {};
+  if (!zero) {
+    src += 36 * tid;
+    const u32x4 x = reinterpret_cast<const u32x4_a4*>(src)[0], y = reinterpret_cast<const u32x4_a4*>(src)[1];
+    const uint32_t w[9] = {x.x, x.y, x.z, x.w, y.x, y.y, y.z, y.w, reinterpret_cast<const uint32_t*>(src)[8]};
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      o[i] = __builtin_bit_cast(u32x4, decode_window(w[2 * i], w[2 * i + 1], w[2 * i + 2], (uint32_t)i));
+  }
+  dst += row * ld + col * 8;
+#pragma unroll
+  for (int i = 0; i < 4; i++) *reinterpret_cast<u32x4*>(dst + i * ld) = o[i];
+}
+
 }  // namespace rl
 
 extern "C" int rl_qkv_post_gqa(const uint16_t* C, int64_t ldc, int64_t M, int32_t hq, int32_t hkv,
@@ -210,4 +279,37 @@ extern "C" int rl_qkv_post(const uint16_t* C, int64_t ldc, int64_t M, int32_t he
                            const uint16_t* sin, const uint16_t* wq, const uint16_t* wk, uint8_t* q_tiles,
                            uint8_t* kv_tiles, uint16_t* q, uint16_t* k, uint16_t* v, void* stream) {
   return rl_qkv_post_gqa(C, ldc, M, heads, heads, cos, sin, wq, wk, q_tiles, kv_tiles, q, k, v, stream);
+}
+
+extern "C" int rl_attn_tiles(const uint8_t* q_tiles, int32_t hq, int64_t q_all, int64_t q_first, int64_t q_count,
+                             int64_t nq, uint16_t* q, const uint8_t* kv0, int64_t all0, int64_t first0, int64_t count0,
+                             const uint8_t* kv1, int64_t all1, int64_t first1, int64_t count1, int32_t hkv, uint16_t* k,
+                             uint16_t* vt, void* stream) {
+  using namespace rl;
+  if (hq < 1 || hq > 1024 || hkv < 1 || hkv > 1024) return fail(RL_ERR_SHAPE, "heads %d / %d: need 1..1024", hq, hkv);
+  constexpr int64_t kMax = 1 << 18;  // tiles per head: 2^24 tokens
+  if (nq < 64 || nq % 64 || nq > 64 * kMax) return fail(RL_ERR_SHAPE, "nq %lld: need a multiple of 64", (long long)nq);
+  if (q_first < 0 || q_count < 1 || q_count > nq / 64 || q_all > kMax || q_first > q_all - q_count)
+    return fail(RL_ERR_SHAPE, "Q tiles %lld + %lld of %lld", (long long)q_first, (long long)q_count, (long long)q_all);
+  if (first0 < 0 || count0 < 1 || all0 > kMax || first0 > all0 - count0)
+    return fail(RL_ERR_SHAPE, "KV tiles %lld + %lld of %lld", (long long)first0, (long long)count0, (long long)all0);
+  if (count1 && (first1 < 0 || count1 < 1 || all1 > kMax || first1 > all1 - count1))
+    return fail(RL_ERR_SHAPE, "second KV tiles %lld + %lld of %lld", (long long)first1, (long long)count1,
+                (long long)all1);
+  if (count0 + count1 > kMax) return fail(RL_ERR_SHAPE, "%lld KV tiles", (long long)(count0 + count1));
+  const int64_t nwg = hq * (nq / 64) + 2 * (int64_t)hkv * (count0 + count1);
+  if (nwg > ((int64_t)1 << 31) - 1) return fail(RL_ERR_SHAPE, "more than 2^31 tiles");
+  if (!q_tiles || !q || !kv0 || !k || !vt || (count1 && !kv1)) return fail(RL_ERR_NULL, "a buffer is NULL");
+  if (((uintptr_t)q_tiles | (uintptr_t)kv0 | (uintptr_t)kv1) % 4 || ((uintptr_t)q | (uintptr_t)k | (uintptr_t)vt) % 16)
+    return fail(RL_ERR_ALIGN, "tiles must be 4-byte, q / k / vt 16-byte aligned");
+  int s;
+  if ((s = check_device())) return s;
+  TilesArgs a;
+  a.q_tiles = q_tiles; a.hq = hq; a.q_all = (int32_t)q_all; a.q_t0 = (int32_t)q_first; a.q_n = (int32_t)q_count;
+  a.q_out = (int32_t)(nq / 64); a.q = q;
+  a.kv[0] = kv0; a.kv_all[0] = (int32_t)all0; a.kv_t0[0] = (int32_t)first0; a.kv_n[0] = (int32_t)count0;
+  a.kv[1] = kv1; a.kv_all[1] = (int32_t)all1; a.kv_t0[1] = (int32_t)first1; a.kv_n[1] = (int32_t)count1;
+  a.hkv = hkv; a.k = k; a.vt = vt;
+  hipLaunchKernelGGL(attn_tiles_kernel, dim3((unsigned)nwg), dim3(kQkvThreads), 0, static_cast<hipStream_t>(stream), a);
+  return launch_status("rl_attn_tiles");
 }

@@ -431,3 +431,29 @@ def attention(q, k, vt, nkv=None, lim=None, out=None, h0=0, quantize_out=False, 
                                     _ptr(out), out.stride(0), h0, 1 if quantize_out else 0, _ptr(ws), max(nbytes, 0),
                                     _stream(q)))
     return out
+
+
+def attn_tiles(q_tiles, heads, q_all, q_first, q_count, nq, kv, kv_heads):
+    """Packed 64-token tiles -> q (heads, nq, 128), k (kv_heads, nk, 128), vt (kv_heads, 128, nk) bf16, exactly. Q: tiles
+    q_first .. + q_count of q_all per head, rows past them zero. kv: one or two (buffer, tiles per head, first, count)
+    ranges of [head][tile][K | V] buffers, joined along the keys. See rl_attn_tiles in include/rlbfp.h."""
+    (b0, all0, f0, n0), (b1, all1, f1, n1) = (list(kv) + [(None, 0, 0, 0)])[:2]
+    nk = 64 * (n0 + n1)
+    z = lambda *shape: torch.empty(shape, dtype=torch.bfloat16, device=q_tiles.device)
+    q, k, vt = z(heads, nq, 128), z(kv_heads, nk, 128), z(kv_heads, 128, nk)
+    L.check(L.lib().rl_attn_tiles(_ptr(q_tiles), heads, q_all, q_first, q_count, nq, _ptr(q), _ptr(b0), all0, f0, n0,
+                                  _ptr(b1), all1, f1, n1, kv_heads, _ptr(k), _ptr(vt), _stream(q_tiles)))
+    return q, k, vt
+
+
+def attention_packed(q, k, vt, out, o_rows, o_cols, h0=0, rows=None, nkv=None, lim=None):
+    """attention() with fewer K / V heads than query heads allowed, O written as bfp16 blocks into rows 0 .. rows - 1,
+    columns (h0 + h) * 128 .. of the A-layout stream `out` (uint8) of an (o_rows, o_cols) matrix; the operands are
+    attn_tiles' outputs. See rl_attention_packed in include/rlbfp.h."""
+    heads, nq = q.shape[:2]
+    hkv, nk = k.shape[:2]
+    nbytes = L.lib().rl_attention_workspace_bytes(heads, nq, nk)
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=q.device) if nbytes > 0 else None
+    L.check(L.lib().rl_attention_packed(_ptr(q), _ptr(k), _ptr(vt), heads, hkv, nq, nk, nk if nkv is None else nkv,
+                                        _ptr(lim), _ptr(out), o_rows, o_cols, h0, nq if rows is None else rows,
+                                        _ptr(ws), max(nbytes, 0), _stream(q)))

@@ -197,6 +197,19 @@ def _write_c_tiles(out, o, heads, nq):
     out.reshape(-1).copy_(t.permute(0, 1, 2, 5, 3, 6, 4, 7).reshape(-1).to(torch.bfloat16))
 
 
+def _tile_range(buf, heads, t_all, t0, n, per=1):
+    """Whether tiles t0 .. t0 + n - 1 of every head can be decoded in place from buf ([head][t_all][per tiles])."""
+    return ops.stream_buffer(buf, torch.uint8, heads * t_all * per * TILE9) and 0 <= t0 and 1 <= n <= t_all - t0
+
+
+def _a_buffer(out, rows_all, cols_all):
+    """Whether `out` can be written in place as the A-layout stream of a (rows_all, cols_all) matrix (a longer buffer
+    may hold more rows)."""
+    return out.device.type == "cuda" and out.dtype == torch.uint8 and out.is_contiguous() and \
+        out.data_ptr() % 16 == 0 and rows_all % 128 == 0 and cols_all % 64 == 0 and \
+        out.numel() >= ops.packed_bytes(rows_all, cols_all) and out.numel() % 9 == 0
+
+
 def run_artifact(meta, args):
     """Run one attention artifact's contract on its NPU buffers (uint8 bfp16 streams, written in place):
       attn32 / attn32o: [Q, KV, O] or, with KVSPLIT, [Q, KV target, KV prefix, O] (attn_design.py:131-281);
@@ -221,14 +234,22 @@ def run_artifact(meta, args):
     q_buf, kv_bufs, o_buf = args[0], list(args[1:-1]), args[-1]
     if len(kv_bufs) != len(geo):
         raise ValueError(f"{len(geo) + 2} buffers expected")
-    q = _q_tiles(q_buf, H, meta.get("QT") or nqt, meta.get("Q0", 0), nqt)
+    oa = bool(meta.get("OA"))
+    q_all, q0 = meta.get("QT") or nqt, meta.get("Q0", 0)
+    oh, h0 = meta.get("OHEADS", 32), meta.get("H0", 0)
+    if oa and nqt % 2 == 0 and 0 <= h0 <= oh - H and _tile_range(q_buf, H, q_all, q0, nqt) and \
+            all(_tile_range(b, H, t_all, t0, n, 2) for b, (t_all, t0), n in zip(kv_bufs, geo, parts)) and \
+            _a_buffer(o_buf, nqt * 64, oh * D):
+        q, k, vt = ops.attn_tiles(q_buf, H, q_all, q0, nqt, nqt * 64,
+                                  [(b, t_all, t0, n) for b, (t_all, t0), n in zip(kv_bufs, geo, parts)], H)
+        ops.attention_packed(q, k, vt, o_buf, nqt * 64, oh * D, h0=h0, nkv=meta.get("NKV") or nk)
+        return
+    q = _q_tiles(q_buf, H, q_all, q0, nqt)
     ks, vs = zip(*(_kv_tiles(b, H, t_all, t0, n) for b, (t_all, t0), n in zip(kv_bufs, geo, parts)))
     k = torch.cat(ks, 1).to(torch.bfloat16).contiguous()
     vt = torch.cat(vs, 1).transpose(1, 2).to(torch.bfloat16).contiguous()
-    oa = bool(meta.get("OA"))
     o = ops.attention(q.contiguous(), k, vt, nkv=meta.get("NKV") or nk, quantize_out=oa)
     if oa:
-        oh, h0 = meta.get("OHEADS", 32), meta.get("H0", 0)
         _write_a_rows(o_buf, o, nqt * 64, oh * D, h0 * D)
     else:
         _write_c_tiles(o_buf, o.reshape(nqt * 64, H, D).permute(1, 0, 2), H, nqt * 64)
@@ -239,16 +260,22 @@ def _run_small(meta, Q, LIM, KV, O):
     buffer; O rows 0..63 of a_layout((128, OHEADS * 128), 128, 64)."""
     H = meta.get("H", 32)
     nkt = meta["NK"] // 64
-    q = _q_tiles(Q, H, 1, 0, 1)
+    pt, p0, oh, h0 = meta.get("PT") or nkt, meta.get("P0", 0), meta.get("OHEADS", 32), meta.get("H0", 0)
     lim = LIM.reshape(-1)[:4 * 64].view(torch.int32)
-    k, v = _kv_tiles(KV, H, meta.get("PT") or nkt, meta.get("P0", 0), nkt)
-    qp = torch.zeros((H, 128, D), dtype=torch.bfloat16, device=Q.device)
-    qp[:, :64] = q
     lp = torch.zeros(128, dtype=torch.int32, device=Q.device)
     lp[:64] = lim.clamp(0, meta["NK"] - 1)
+    if _tile_range(Q, H, 1, 0, 1) and _tile_range(KV, H, pt, p0, nkt, 2) and 0 <= h0 <= oh - H and \
+            _a_buffer(O, 128, oh * D):
+        q, k, vt = ops.attn_tiles(Q, H, 1, 0, 1, 128, [(KV, pt, p0, nkt)], H)
+        ops.attention_packed(q, k, vt, O, 128, oh * D, h0=h0, rows=64, lim=lp)
+        return
+    q = _q_tiles(Q, H, 1, 0, 1)
+    k, v = _kv_tiles(KV, H, pt, p0, nkt)
+    qp = torch.zeros((H, 128, D), dtype=torch.bfloat16, device=Q.device)
+    qp[:, :64] = q
     o = ops.attention(qp, k.to(torch.bfloat16).contiguous(), v.transpose(1, 2).to(torch.bfloat16).contiguous(),
                       lim=lp, quantize_out=True)
-    _write_a_rows(O, o[:64], 128, meta.get("OHEADS", 32) * D, meta.get("H0", 0) * D)
+    _write_a_rows(O, o[:64], 128, oh * D, h0 * D)
 
 
 def _run_causal(meta, Q, KV, O):
@@ -260,6 +287,12 @@ def _run_causal(meta, Q, KV, O):
     hq, hkv = Q.numel() // (T * TILE9), KV.numel() // (T * 2 * TILE9)
     n = nqt * 64
     nq = -(-n // 128) * 128
+    if hkv and hq % hkv == 0 and _tile_range(Q, hq, T, 0, nqt) and _tile_range(KV, hkv, T, 0, nqt, 2) and \
+            _a_buffer(O, M, hq * D):
+        q, k, vt = ops.attn_tiles(Q, hq, T, 0, nqt, nq, [(KV, T, 0, nqt)], hkv)
+        lim = torch.arange(nq, dtype=torch.int32, device=Q.device)
+        ops.attention_packed(q, k, vt, O, M, hq * D, rows=n, lim=lim)
+        return
     q = torch.zeros((hq, nq, D), dtype=torch.bfloat16, device=Q.device)
     q[:, :n] = _q_tiles(Q, hq, T, 0, nqt)
     k, v = _kv_tiles(KV, hkv, T, 0, nqt)

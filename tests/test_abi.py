@@ -257,3 +257,19 @@ def test_ln_stream_rejects_before_any_gpu_call():
     assert f(16, None, 2, 16, 0, 0, 16, 16, 512, 1024, None) == L.RL_ERR_ARG
     assert f(16, None, 0, 16, 0, 0, None, 16, 512, 1024, None) == L.RL_ERR_NULL
     assert f(16, None, 0, 16, 0, 0, 16, 8, 512, 1024, None) == L.RL_ERR_ALIGN
+
+
+def test_attention_packed_rejects_before_any_gpu_call():
+    f = L.lib().rl_attention_packed
+    call = lambda heads=4, hkv=2, nq=256, o_rows=256, o_cols=512, h0=0, rows=256, o=16: f(
+        16, 16, 16, heads, hkv, nq, 128, 128, None, o, o_rows, o_cols, h0, rows, None, 0, None)
+    assert call(hkv=3) == L.RL_ERR_SHAPE and call(hkv=0) == L.RL_ERR_SHAPE
+    assert call(o_rows=192, rows=192) == L.RL_ERR_SHAPE and call(rows=8) == L.RL_ERR_SHAPE
+    assert call(rows=512, o_rows=512) == L.RL_ERR_SHAPE and call(o_rows=128) == L.RL_ERR_SHAPE
+    assert call(h0=1) == L.RL_ERR_ALIGN and call(o=None) == L.RL_ERR_NULL and call(o=8) == L.RL_ERR_ALIGN
+    g = L.lib().rl_attn_tiles
+    tiles = lambda q=(4, 1, 3), nq=192, kv=(5, 0, 5), kv1=(0, 0, 0), b1=None: g(
+        16, 2, *q, nq, 16, 16, *kv, b1, *kv1, 1, 16, 16, None)
+    assert tiles(q=(4, 2, 3)) == L.RL_ERR_SHAPE and tiles(nq=128) == L.RL_ERR_SHAPE
+    assert tiles(kv=(5, 1, 5)) == L.RL_ERR_SHAPE and tiles(kv=(5, -1, 5)) == L.RL_ERR_SHAPE
+    assert tiles(kv1=(3, 1, 3), b1=16) == L.RL_ERR_SHAPE and tiles(kv1=(3, 0, 3)) == L.RL_ERR_NULL

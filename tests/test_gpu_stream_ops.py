@@ -5,10 +5,11 @@ import numpy as np
 import pytest
 import torch
 
+from oracle import attn as A
 from oracle import bfp16 as F
 from oracle import gemm as G
 from oracle import ln as LN
-from rlbfp import forward, layouts, ops, run_ln
+from rlbfp import forward, layouts, ops, run_attn, run_ln
 
 pytestmark = pytest.mark.gpu
 
@@ -68,3 +69,110 @@ def test_ln_stream_general_form(dev):
         run_ln.ln_fused("glue-ln-m512-s1", X, B, p, x2, A)
         assert torch.equal(x2, xo)
         assert (layouts.from_bfp16(A) == layouts.from_bfp16(ao)).float().mean() > 0.999
+
+
+# ---- attention on packed tiles ------------------------------------------------------------------------------------
+
+def tiles(rng, heads, t, kv=False):
+    """Random Q ([head][tile]) or KV ([head][tile][K | V]) tiles and their decoded values (heads, 64 t, 128)."""
+    mk = lambda: rng.standard_normal((heads, 64 * t, 128)).astype(np.float32)
+    rows = lambda x, h, i: x[h, 64 * i:64 * i + 64]
+    if not kv:
+        q = mk() * A.C_LOG2
+        raw = [F.to_bfp16(F.a_layout(rows(q, h, i), 64, 128)) for h in range(heads) for i in range(t)]
+        return tt(np.concatenate(raw), torch.uint8), F.quantize_rows(q.reshape(-1, 128)).reshape(q.shape)
+    k, v = mk(), mk()
+    raw = []
+    for h in range(heads):
+        for i in range(t):
+            raw += [F.to_bfp16(F.b_layout(np.ascontiguousarray(rows(k, h, i).T), 128, 64)),
+                    F.to_bfp16(F.b_layout(rows(v, h, i), 64, 128))]
+    vq = F.quantize_rows(np.ascontiguousarray(v.transpose(0, 2, 1)).reshape(-1, 64 * t)).reshape(heads, 128, 64 * t)
+    return tt(np.concatenate(raw), torch.uint8), (F.quantize_rows(k.reshape(-1, 128)).reshape(k.shape),
+                                                  np.ascontiguousarray(vq.transpose(0, 2, 1)))
+
+
+@pytest.mark.parametrize("hq,hkv,qa,q0,qn,nq,kv", [
+    (2, 2, 2, 0, 2, 128, [(3, 0, 3)]), (3, 1, 5, 1, 3, 256, [(4, 2, 1), (7, 3, 4)]), (1, 2, 1, 0, 1, 128, [(1, 0, 1)])])
+def test_attn_tiles(dev, hq, hkv, qa, q0, qn, nq, kv):
+    """Tile ranges of one or two K / V buffers, query rows past the range: the exact values."""
+    rng = np.random.default_rng(hq + nq)
+    qb, qv = tiles(rng, hq, qa)
+    bufs = [tiles(rng, hkv, t, kv=True) for t, _, _ in kv]
+    q, k, vt = ops.attn_tiles(qb, hq, qa, q0, qn, nq, [(b[0], *g) for b, g in zip(bufs, kv)], hkv)
+    ref_q = np.zeros((hq, nq, 128), np.float32)
+    ref_q[:, :64 * qn] = qv[:, 64 * q0:64 * (q0 + qn)]
+    cut = lambda x, g: x[:, 64 * g[1]:64 * (g[1] + g[2])]
+    np.testing.assert_array_equal(q.float().cpu().numpy(), ref_q)
+    np.testing.assert_array_equal(k.float().cpu().numpy(), np.concatenate([cut(b[1][0], g) for b, g in zip(bufs, kv)], 1))
+    np.testing.assert_array_equal(vt.float().cpu().numpy().transpose(0, 2, 1),
+                                  np.concatenate([cut(b[1][1], g) for b, g in zip(bufs, kv)], 1))
+
+
+def check_o(got, ref):
+    """Packed O against float64: 1e-2 of the largest value (P in bf16, O in bfp16), correlation above 0.9999."""
+    assert G.rel_err(got, ref) <= 1e-2 and G.corr(got, ref) > 0.9999
+
+
+@pytest.mark.parametrize("H,OH,H0,nqt,nk,pad", [(2, 2, 0, 4, 5, 13), (1, 3, 1, 2, 33, 64), (3, 4, 1, 6, 2, 0),
+                                                (65, 65, 0, 16, 2, 1)])
+def test_attn_artifact(dev, H, OH, H0, nqt, nk, pad):
+    """Whole tasks and tasks split along the keys, 4- and 8-wave workgroups, an O wider than the heads, padded keys (a
+    whole tile of them too): against float64 and against the general form; other columns of O stay."""
+    rng = np.random.default_rng(H + nk)
+    qb, qv = tiles(rng, H, nqt)
+    kb, (kd, vd) = tiles(rng, H, nk, kv=True)
+    meta = {"family": "attn32o", "H": H, "QN": nqt, "NK": 64 * nk, "NKV": 64 * nk - pad, "OA": 1, "OHEADS": OH, "H0": H0}
+    M = 64 * nqt
+    o = torch.full((M * OH * 128 // 8 * 9,), 5, dtype=torch.uint8, device="cuda")
+    run_attn.run_artifact(meta, [qb, kb, o])
+    full = layouts.from_bfp16_a_layout(o, M, OH * 128)
+    got = full.cpu().numpy().reshape(M, OH, 128).transpose(1, 0, 2)
+    hs = list(range(H)) if H < 8 else [0, 31, 64]
+    check_o(got[[H0 + h for h in hs]], A.attention_ref(qv[hs], kd[hs], vd[hs], nkv=64 * nk - pad))
+    rest = torch.full_like(o, 5)
+    untouched = layouts.from_bfp16_a_layout(rest, M, OH * 128).reshape(M, OH, 128)
+    keep = [h for h in range(OH) if not H0 <= h < H0 + H]
+    assert torch.equal(full.reshape(M, OH, 128)[:, keep], untouched[:, keep])
+    # the general form re-encodes bf16 values, which only blocks led by -128 change
+    q, k, vt = ops.attn_tiles(qb, H, nqt, 0, nqt, M, [(kb, nk, 0, nk)], H)
+    o16 = ops.attention(q, k, vt, nkv=64 * nk - pad, quantize_out=True)
+    same = full.reshape(M, OH * 128)[:, H0 * 128:(H0 + H) * 128] == o16.float()
+    assert same.all()
+
+
+@pytest.mark.parametrize("hq,hkv,M,nqt", [(4, 2, 256, 3), (8, 1, 512, 8), (32, 8, 1536, 17), (64, 64, 1280, 20)])
+def test_causal_artifact(dev, hq, hkv, M, nqt):
+    """Grouped-query heads, an odd number of query tiles, rows past them left alone, more tasks than workgroups."""
+    rng = np.random.default_rng(hq + nqt)
+    T, n = M // 64, 64 * nqt
+    qb, qv = tiles(rng, hq, T)
+    kb, (kd, vd) = tiles(rng, hkv, T, kv=True)
+    o = torch.full((M * hq * 128 // 8 * 9,), 5, dtype=torch.uint8, device="cuda")
+    run_attn.run_artifact({"family": "causal", "M": M, "NQT": nqt}, [qb, kb, o])
+    full = layouts.from_bfp16_a_layout(o, M, hq * 128)
+    got = full.cpu().numpy().reshape(M, hq, 128).transpose(1, 0, 2)
+    g = hq // hkv
+    for h in (0, hq // 2, hq - 1):
+        ref = A.attention_ref(qv[h:h + 1, :n], kd[h // g:h // g + 1, :n], vd[h // g:h // g + 1, :n], lim=np.arange(n))
+        check_o(got[h:h + 1, :n], ref)
+        # query 0 sees key 0 only: O is that V row (blocks of 8 keys) rounded to blocks of 8 dims
+        np.testing.assert_array_equal(got[h, :1], F.quantize_rows(vd[h // g, :1]))
+    keep = layouts.from_bfp16_a_layout(torch.full_like(o, 5), M, hq * 128)
+    assert torch.equal(full[n:], keep[n:])
+
+
+@pytest.mark.parametrize("H,NQ,NK,split", [(2, 256, 1024, True), (3, 384, 640, False), (300, 256, 128, True)])
+def test_limits_clip(dev, H, NQ, NK, split):
+    """Limits that let a workgroup skip key blocks (sorted, and below zero: a query that sees nothing gives 0)."""
+    rng = np.random.default_rng(H)
+    mk = lambda n: F.bf16_round(rng.standard_normal((H, n, 128)).astype(np.float32))
+    q, k, v = F.bf16_round(mk(NQ) * np.float32(A.C_LOG2)), mk(NK), mk(NK)
+    lim = np.sort(rng.integers(-40, NK, NQ)).astype(np.int32)
+    lim[:130] = -1
+    o = ops.attention(tt(q, torch.bfloat16), tt(k, torch.bfloat16),
+                      tt(v.transpose(0, 2, 1), torch.bfloat16), nkv=NK - 7, lim=tt(lim, torch.int32), split=split)
+    got = o.float().cpu().numpy().reshape(NQ, H, 128).transpose(1, 0, 2)
+    assert (got[:, :130] == 0).all()
+    hs = [0, H // 2, H - 1]
+    check_o(got[hs], A.attention_ref(q[hs], k[hs], v[hs], nkv=NK - 7, lim=lim))
