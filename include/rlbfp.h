@@ -251,6 +251,14 @@ int rl_qkv_post_gqa(const uint16_t *C, int64_t ldc, int64_t M, int32_t hq, int32
                     const uint16_t *sin, const uint16_t *wq, const uint16_t *wk, uint8_t *q_tiles, uint8_t *kv_tiles,
                     uint16_t *q, uint16_t *k, uint16_t *v, void *stream);
 
+/* rl_qkv_post_gqa on the artifact's own buffers (redline/run_qkv.py:52-82): C is the QKV GEMM's C stream of (M, (hq + 2
+ * hkv) * 128) values, bfp16 blocks (c_packed) or bf16, in the order c_layout_atb(., 128, 128); tabs is the qkv_tables
+ * buffer, (M / 64, 8448) bf16: per 64-row tile cos / sin in the order of the tile's 8 x 8 input blocks, then wq and wk
+ * (those of tile 0 are used). Outputs: q_tiles and kv_tiles as above (both required), the same bytes. M % 512 == 0,
+ * columns % 1024 == 0; every pointer 16-byte aligned. */
+int rl_qkv_post_stream(const void *C, int32_t c_packed, int64_t M, int32_t hq, int32_t hkv, const uint16_t *tabs,
+                       uint8_t *q_tiles, uint8_t *kv_tiles, void *stream);
+
 /* ---- attention over the QKV post pass's output -------------------------------------------------------------------
  * Per head h and query i: O[i][(h0 + h) * 128 + d] = sum_j P[i][j] V[j][d], P = 2^(S - max) / sum over the visible
  * keys, S = Q K^T. Q carries the score scale log2(e)/sqrt(128) (as rl_qkv_post's wq does), so S is in log2 units.

@@ -68,6 +68,26 @@ __device__ __forceinline__ void stage_block(uint8_t* stage, int pos, uint32_t E,
   for (int e = 0; e < 8; e++) p[1 + e] = (uint8_t)(int8_t)q[e];
 }
 
+// One token's 8 dims of a head (the other 15 blocks in the lanes of its row of 16): rope(x / rms * w) as float32 bits
+__device__ __forceinline__ void rms_rope8(const float (&xf)[8], const float (&wf)[8], uint2 cr, uint2 sr,
+                                          uint32_t (&u)[8]) {
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; e++) ss = fmaf(xf[e], xf[e], ss);
+  ss = row16_sum(ss);  // the token's 16 lanes
+  const float inv = __builtin_amdgcn_rsqf(ss / (float)kHeadDim + 1e-6f);
+  const float c4[4] = {__uint_as_float(cr.x << 16), __uint_as_float(cr.x & 0xFFFF0000u),
+                       __uint_as_float(cr.y << 16), __uint_as_float(cr.y & 0xFFFF0000u)};
+  const float s4[4] = {__uint_as_float(sr.x << 16), __uint_as_float(sr.x & 0xFFFF0000u),
+                       __uint_as_float(sr.y << 16), __uint_as_float(sr.y & 0xFFFF0000u)};
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const float ev = xf[2 * i] * inv * wf[2 * i], od = xf[2 * i + 1] * inv * wf[2 * i + 1];
+    u[2 * i] = __float_as_uint(ev * c4[i] - od * s4[i]);
+    u[2 * i + 1] = __float_as_uint(ev * s4[i] + od * c4[i]);
+  }
+}
+
 // TILES / NATIVE: whether any tile / any head-major bf16 output is requested (the other's work is compiled out).
 template <bool TILES, bool NATIVE>
 __global__ __launch_bounds__(kQkvThreads) void qkv_post_kernel(QkvArgs a) {
@@ -114,25 +134,10 @@ __global__ __launch_bounds__(kQkvThreads) void qkv_post_kernel(QkvArgs a) {
       const int64_t row = row0 + r;
       float xf[8];
       unpack8f(xr[pass], xf);
-      float ss = 0.f;
-#pragma unroll
-      for (int e = 0; e < 8; e++) ss = fmaf(xf[e], xf[e], ss);
-      ss = row16_sum(ss);  // the token's 16 lanes
-      const float inv = __builtin_amdgcn_rsqf(ss / (float)kHeadDim + 1e-6f);
-      const uint2 cr = cr4[pass], sr = sr4[pass];
-      const float c4[4] = {__uint_as_float(cr.x << 16), __uint_as_float(cr.x & 0xFFFF0000u),
-                           __uint_as_float(cr.y << 16), __uint_as_float(cr.y & 0xFFFF0000u)};
-      const float s4[4] = {__uint_as_float(sr.x << 16), __uint_as_float(sr.x & 0xFFFF0000u),
-                           __uint_as_float(sr.y << 16), __uint_as_float(sr.y & 0xFFFF0000u)};
       uint32_t u[8];
       int32_t q[8];
       u32x4 bw;
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const float ev = xf[2 * i] * inv * wf[2 * i], od = xf[2 * i + 1] * inv * wf[2 * i + 1];
-        u[2 * i] = __float_as_uint(ev * c4[i] - od * s4[i]);
-        u[2 * i + 1] = __float_as_uint(ev * s4[i] + od * c4[i]);
-      }
+      rms_rope8(xf, wf, cr4[pass], sr4[pass], u);
       const uint32_t E = encode_block(u, q, bw);
       if (nat) *reinterpret_cast<u32x4*>(nat + (((int64_t)h * a.M + row) * kHeadDim + bc * 8)) = bw;
       // a_layout(64, 128) for Q and b_layout(K^T, 128, 64) for K order a tile's blocks the same way:
@@ -165,6 +170,122 @@ __global__ __launch_bounds__(kQkvThreads) void qkv_post_kernel(QkvArgs a) {
     }
   }
   if (!tiles) return;
+  __syncthreads();
+  const int64_t T = a.M / kTileTokens;
+  uint8_t* dst = part == 0 ? a.q_tiles + ((int64_t)h * T + t) * kTile9
+                           : a.kv_tiles + (((int64_t)h * T + t) * 2 + (part - 1)) * kTile9;
+  for (int c = tid; c < kTile9 / 16; c += kQkvThreads)
+    *reinterpret_cast<u32x4*>(dst + 16 * c) = *reinterpret_cast<const u32x4*>(&stage[16 * c]);
+}
+
+// ---- the same pass on the artifact's own buffers ----------------------------------------------------------------------
+//
+// C is the QKV GEMM's C stream (bfp16, or bf16 in that element order), cos / sin come from the NPU kernel's table
+// (redline/run_qkv.py:52-64). In both orders the 64 x 128 tile of one head is contiguous: 4 row bands x 8 column
+// bands x (2 x 2) 8 x 8 blocks, 9216 bytes of bfp16 (16 KB of bf16, 16 KB of table), so a workgroup reads one run of C
+// and one of the table and writes one run of tiles. Thread (column block bc = tid & 15, row quad) takes rows 4 quad ..
+// + 3 of one 8-dim block: four consecutive blocks of C (36 or 64 bytes), of the table (32 + 32) and of the output tile
+// (36 bytes). A token's 16 blocks sit in 16 neighbouring lanes, as in qkv_post_kernel. V goes through a 16 KB LDS tile
+// of decoded values, read down the columns.
+// HBM-bound: 9/8 (or 2) bytes read and 9/8 written per value. It replaces a decode pass, index passes over the table and
+// the row-major kernel: at 4096 x 12288 this kernel takes 30 us (113 MB of tiles and 34 MB of table re-read by every
+// head, from L2), and the attention step that holds it went from 1155 to 1025 us.
+struct QkvStreamArgs {
+  const void* C;
+  int32_t n_cols;
+  int32_t hq, hkv;
+  int64_t M;
+  const uint16_t* tabs;  // (M / 64, kTabLen)
+  uint8_t* q_tiles;
+  uint8_t* kv_tiles;
+};
+constexpr int kTabLen = 128 * 64 + 2 * 128;
+
+// Four blocks' values, row i's block in u[i] (float32 bits) -> their 36 bytes at p
+__device__ __forceinline__ void encode_store4(uint8_t* p, const uint32_t (&u)[4][8]) {
+  uint32_t E[4], ql[4], qh[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    int32_t q[8];
+    u32x4 bw;
+    E[i] = encode_block(u[i], q, bw);
+    ql[i] = (q[0] & 0xFFu) | ((q[1] & 0xFFu) << 8) | ((q[2] & 0xFFu) << 16) | ((uint32_t)q[3] << 24);
+    qh[i] = (q[4] & 0xFFu) | ((q[5] & 0xFFu) << 8) | ((q[6] & 0xFFu) << 16) | ((uint32_t)q[7] << 24);
+  }
+  store_blocks4(p, E, ql, qh);
+}
+
+// PACKED: C as bfp16 blocks, else bf16
+template <bool PACKED>
+__global__ __launch_bounds__(kQkvThreads) void qkv_stream_kernel(QkvStreamArgs a) {
+  typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
+  constexpr int kVRow = kHeadDim + 8;  // LDS row of V values: 16 bytes of padding
+  __shared__ __attribute__((aligned(16))) uint8_t stage[kTile9];
+  __shared__ __attribute__((aligned(16))) uint16_t vals[kTileTokens * kVRow];
+  const int tid = threadIdx.x, bc = tid & 15, quad = tid >> 4;  // quad: row 4 quad of the 64
+  const int per_tile = a.hq + 2 * a.hkv;
+  const int t = blockIdx.x / per_tile, j = blockIdx.x - t * per_tile;
+  int part, h;
+  if (a.hq == a.hkv) {
+    part = j % 3; h = j / 3;
+  } else if (j < a.hq) {
+    part = 0; h = j;
+  } else {
+    part = 1 + ((j - a.hq) & 1); h = (j - a.hq) >> 1;
+  }
+  const int col128 = part == 0 ? h : a.hq + (part - 1) * a.hkv + h;
+  // blocks of a tile: row band, column band, row half, column half, row in 8
+  const int loc = ((((quad >> 2) * 8 + (bc >> 1)) * 2 + ((quad >> 1) & 1)) * 2 + (bc & 1)) * 8 + (quad & 1) * 4;
+  // 64-row tile t of 128-column group col128: row group t / 8, then column groups, 128-row groups, 16-row bands
+  const int64_t blk = ((int64_t)(t >> 3) * (a.n_cols >> 7) + col128) * 8192 + (t & 7) * 1024 + loc;
+  u32x4 x[4];
+  if constexpr (PACKED) {
+    const uint8_t* src = static_cast<const uint8_t*>(a.C) + 9 * blk;
+    const u32x4 b0 = reinterpret_cast<const u32x4_a4*>(src)[0], b1 = reinterpret_cast<const u32x4_a4*>(src)[1];
+    const uint32_t w[9] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w, reinterpret_cast<const uint32_t*>(src)[8]};
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      x[i] = __builtin_bit_cast(u32x4, decode_window(w[2 * i], w[2 * i + 1], w[2 * i + 2], (uint32_t)i));
+  } else {
+    const u32x4* src = reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(a.C) + 8 * blk);
+#pragma unroll
+    for (int i = 0; i < 4; i++) x[i] = src[i];
+  }
+  uint32_t u[4][8];
+  int pos;
+  if (part < 2) {
+    // the table's block: 8 rows x 4 cos, then 8 rows x 4 sin; its index is loc / 8
+    const uint16_t* tab = a.tabs + (int64_t)t * kTabLen + (loc >> 3) * 64 + (quad & 1) * 16;
+    uint2 cr4[4], sr4[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      cr4[i] = *reinterpret_cast<const uint2*>(tab + 4 * i);
+      sr4[i] = *reinterpret_cast<const uint2*>(tab + 32 + 4 * i);
+    }
+    float wf[8];
+    unpack8f(*reinterpret_cast<const u32x4*>(a.tabs + kTabLen - 256 + part * 128 + bc * 8), wf);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      float xf[8];
+      unpack8f(x[i], xf);
+      rms_rope8(xf, wf, cr4[i], sr4[i], u[i]);
+    }
+    pos = ((quad >> 2) * 16 + bc) * 16 + (quad & 3) * 4;  // 16-token band, 8-dim block, token
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; i++) *reinterpret_cast<u32x4*>(&vals[(4 * quad + i) * kVRow + 8 * bc]) = x[i];
+    __syncthreads();
+    // thread (dim quad tid & 31, 8-token block tid >> 5): the 8 tokens of dims 4 dq .. + 3
+    const int dq = tid & 31, kb = tid >> 5;
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      const uint2 v = *reinterpret_cast<const uint2*>(&vals[(8 * kb + e) * kVRow + 4 * dq]);
+      u[0][e] = v.x << 16; u[1][e] = v.x & 0xFFFF0000u;
+      u[2][e] = v.y << 16; u[3][e] = v.y & 0xFFFF0000u;
+    }
+    pos = ((dq >> 2) * 8 + kb) * 16 + (dq & 3) * 4;  // 16-dim band, token block, dim
+  }
+  encode_store4(stage + pos * kBlockBytes, u);
   __syncthreads();
   const int64_t T = a.M / kTileTokens;
   uint8_t* dst = part == 0 ? a.q_tiles + ((int64_t)h * T + t) * kTile9
@@ -312,4 +433,29 @@ extern "C" int rl_attn_tiles(const uint8_t* q_tiles, int32_t hq, int64_t q_all, 
   a.hkv = hkv; a.k = k; a.vt = vt;
   hipLaunchKernelGGL(attn_tiles_kernel, dim3((unsigned)nwg), dim3(kQkvThreads), 0, static_cast<hipStream_t>(stream), a);
   return launch_status("rl_attn_tiles");
+}
+
+extern "C" int rl_qkv_post_stream(const void* C, int32_t c_packed, int64_t M, int32_t hq, int32_t hkv,
+                                  const uint16_t* tabs, uint8_t* q_tiles, uint8_t* kv_tiles, void* stream) {
+  using namespace rl;
+  const int64_t n = 128 * ((int64_t)hq + 2 * (int64_t)hkv);
+  int s = rl_validate_qkv_post_gqa(n, M, hq, hkv);
+  if (s) return s;
+  if (M % 512 || n % 1024)
+    return fail(RL_ERR_SHAPE, "M %lld, %lld columns: the C-stream order needs M %% 512 == 0 and columns %% 1024 == 0",
+                (long long)M, (long long)n);
+  if (!C || !tabs || !q_tiles || !kv_tiles) return fail(RL_ERR_NULL, "C, tabs or an output is NULL");
+  if (((uintptr_t)C | (uintptr_t)tabs | (uintptr_t)q_tiles | (uintptr_t)kv_tiles) % 16)
+    return fail(RL_ERR_ALIGN, "C, tabs and the tiles must be 16-byte aligned");
+  if ((s = check_device())) return s;
+  QkvStreamArgs a;
+  a.C = C; a.n_cols = (int32_t)n; a.hq = hq; a.hkv = hkv; a.M = M; a.tabs = tabs; a.q_tiles = q_tiles;
+  a.kv_tiles = kv_tiles;
+  const dim3 grid((unsigned)(M / kTileTokens * (hq + 2 * hkv)));
+  const hipStream_t st = static_cast<hipStream_t>(stream);
+  if (c_packed)
+    hipLaunchKernelGGL(qkv_stream_kernel<true>, grid, dim3(kQkvThreads), 0, st, a);
+  else
+    hipLaunchKernelGGL(qkv_stream_kernel<false>, grid, dim3(kQkvThreads), 0, st, a);
+  return launch_status("rl_qkv_post_stream");
 }

@@ -234,6 +234,23 @@ __device__ __forceinline__ uint32_t quantize_with_exp(uint32_t u, uint32_t E) {
   return decode_bf16_bits(encode_elem(u, E), E);
 }
 
+// Four bfp16 blocks (exponents E[i], q0..q3 in ql[i], q4..q7 in qh[i]) as their 36 consecutive bytes
+// [E0 q0..q7][E1 ...][E2 ...][E3 ...], written as 9 dwords (p is 4-byte aligned: a block index that is a multiple
+// of 4 times 9 bytes)
+__device__ __forceinline__ void store_blocks4(uint8_t* p, const uint32_t (&E)[4], const uint32_t (&ql)[4],
+                                              const uint32_t (&qh)[4]) {
+  uint32_t* w = reinterpret_cast<uint32_t*>(p);
+  w[0] = E[0] | (ql[0] << 8);
+  w[1] = (ql[0] >> 24) | (qh[0] << 8);
+  w[2] = (qh[0] >> 24) | (E[1] << 8) | (ql[1] << 16);
+  w[3] = (ql[1] >> 16) | (qh[1] << 16);
+  w[4] = (qh[1] >> 16) | (E[2] << 16) | (ql[2] << 24);
+  w[5] = (ql[2] >> 8) | (qh[2] << 24);
+  w[6] = (qh[2] >> 8) | (E[3] << 24);
+  w[7] = ql[3];
+  w[8] = qh[3];
+}
+
 // Waits until at most N vector-memory loads of this wave are outstanding (s_waitcnt vmcnt(N), gfx9 encoding).
 template <int N>
 __device__ __forceinline__ void wait_vm() {

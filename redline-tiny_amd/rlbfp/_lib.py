@@ -68,6 +68,7 @@ SIGNATURES = {
     "rl_ln_modulate_stream": (ctypes.c_int, [_P, _P, _I32, _P, _I64, _I32, _P, _P, _I64, _I64, _P]),
     "rl_qkv_post": (ctypes.c_int, [_P, _I64, _I64, _I32, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
     "rl_qkv_post_gqa": (ctypes.c_int, [_P, _I64, _I64, _I32, _I32, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
+    "rl_qkv_post_stream": (ctypes.c_int, [_P, _I32, _I64, _I32, _I32, _P, _P, _P, _P]),
     "rl_attention": (ctypes.c_int, [_P, _P, _P, _I32, _I64, _I64, _I64, _P, _P, _I64, _I32, _I32, _P]),
     "rl_attention_ws": (ctypes.c_int, [_P, _P, _P, _I32, _I64, _I64, _I64, _P, _P, _I64, _I32, _I32, _P, _I64, _P]),
     "rl_attention_workspace_bytes": (ctypes.c_int64, [_I32, _I64, _I64]),

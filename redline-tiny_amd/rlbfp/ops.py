@@ -397,6 +397,13 @@ def qkv_post(C, cos, sin, wq, wk, heads, tiles=True, native=False, kv_heads=None
     return qt, kvt, q, k, v
 
 
+def qkv_post_stream(C, M, heads, kv_heads, tabs, q_tiles, kv_tiles):
+    """qkv_post on the artifact's buffers: C the QKV GEMM's C stream (uint8 bfp16, or flat bf16 in that order), tabs the
+    run_qkv.qkv_tables buffer, the tiles written to q_tiles and kv_tiles. See rl_qkv_post_stream in include/rlbfp.h."""
+    L.check(L.lib().rl_qkv_post_stream(_ptr(C), 1 if C.dtype == torch.uint8 else 0, M, heads, kv_heads, _ptr(tabs),
+                                       _ptr(q_tiles), _ptr(kv_tiles), _stream(C)))
+
+
 # ---------------------------------------------------------------------------------------------------------------
 # attention
 # ---------------------------------------------------------------------------------------------------------------

@@ -111,6 +111,21 @@ def unpack_head(q, kv, h):
     return Q, K, V
 
 
+def _stream_form(cin, tabs, q_out, kv_out, M, T, hq, hkv):
+    """Whether the artifact's buffers can be read and written in place: C a whole C stream (uint8, or flat bf16), the
+    table and the tiles whole, on one device, no output over an input."""
+    n = M * 128 * (hq + 2 * hkv)
+    if not (ops.stream_buffer(cin, torch.uint8, n // 8 * 9) or
+            cin.dim() == 1 and ops.stream_buffer(cin, torch.bfloat16, n)):
+        return False
+    outs, ins = (q_out, kv_out), (cin, tabs)
+    return ops.stream_buffer(tabs, torch.bfloat16, T * TAB) and hq >= 1 and hkv >= 1 and \
+        ops.stream_buffer(q_out, torch.uint8, hq * T * 9216) and \
+        ops.stream_buffer(kv_out, torch.uint8, hkv * T * 2 * 9216) and \
+        all(t.device == cin.device for t in (tabs, *outs)) and \
+        not any(ops.overlaps(o, i) for o in outs for i in ins) and not ops.overlaps(q_out, kv_out)
+
+
 def qkv_post_run(art, cin, tabs, q_out, kv_out):
     """NPU.run("qkv_post", art, [C, TABS, Q, KV]): the QKV-post artifacts' buffer contract (redline/forward.py:246,
     :368; GQA copy: redline/vlm_run.py:433-437, kernels/vlm/qkv_gqa_design.py:1-10), written into the caller's Q
@@ -122,6 +137,9 @@ def qkv_post_run(art, cin, tabs, q_out, kv_out):
     M = 64 * T
     hq, hkv = q_out.numel() // (T * 9216), kv_out.numel() // (T * 2 * 9216)
     n_cols = 128 * (hq + 2 * hkv)
+    if M and M % 512 == 0 and n_cols % 1024 == 0 and _stream_form(cin, tabs, q_out, kv_out, M, T, hq, hkv):
+        ops.qkv_post_stream(cin, M, hq, hkv, tabs, q_out, kv_out)
+        return
     if cin.dtype == torch.uint8:
         C = ops.dequantize(cin.reshape(-1), M, n_cols, order="c_atb", dtype=torch.bfloat16)
     elif cin.dim() == 1:

@@ -273,3 +273,12 @@ def test_attention_packed_rejects_before_any_gpu_call():
     assert tiles(q=(4, 2, 3)) == L.RL_ERR_SHAPE and tiles(nq=128) == L.RL_ERR_SHAPE
     assert tiles(kv=(5, 1, 5)) == L.RL_ERR_SHAPE and tiles(kv=(5, -1, 5)) == L.RL_ERR_SHAPE
     assert tiles(kv1=(3, 1, 3), b1=16) == L.RL_ERR_SHAPE and tiles(kv1=(3, 0, 3)) == L.RL_ERR_NULL
+
+
+def test_qkv_stream_rejects_before_any_gpu_call():
+    f = L.lib().rl_qkv_post_stream
+    assert f(16, 1, 576, 8, 8, 16, 16, 16, None) == L.RL_ERR_SHAPE    # M % 512
+    assert f(16, 1, 512, 8, 2, 16, 16, 16, None) == L.RL_ERR_SHAPE    # 1536 columns
+    assert f(16, 1, 512, 0, 4, 16, 16, 16, None) == L.RL_ERR_SHAPE
+    assert f(16, 1, 512, 8, 8, 16, None, 16, None) == L.RL_ERR_NULL
+    assert f(16, 1, 512, 8, 8, 8, 16, 16, None) == L.RL_ERR_ALIGN

@@ -9,7 +9,7 @@ from oracle import attn as A
 from oracle import bfp16 as F
 from oracle import gemm as G
 from oracle import ln as LN
-from rlbfp import forward, layouts, ops, run_attn, run_ln
+from rlbfp import forward, layouts, ops, run_attn, run_ln, run_qkv
 
 pytestmark = pytest.mark.gpu
 
@@ -176,3 +176,32 @@ def test_limits_clip(dev, H, NQ, NK, split):
     assert (got[:, :130] == 0).all()
     hs = [0, H // 2, H - 1]
     check_o(got[hs], A.attention_ref(q[hs], k[hs], v[hs], nkv=NK - 7, lim=lim))
+
+
+# ---- QKV post on the C stream and the rotary table ----------------------------------------------------------------
+
+@pytest.mark.parametrize("M,hq,hkv", [(512, 8, 8), (1024, 4, 2), (512, 6, 1), (1536, 32, 8)])
+@pytest.mark.parametrize("packed", [True, False])
+def test_qkv_stream(dev, monkeypatch, M, hq, hkv, packed):
+    """The tiles equal those of the general form (C and the table to row-major order, then rl_qkv_post) byte for byte:
+    the same float32 arithmetic on the same values; blocks of zeros and of extreme exponents among them."""
+    rng = np.random.default_rng(M + hq)
+    n = 128 * (hq + 2 * hkv)
+    C = (rng.standard_normal((M, n)) * 2).astype(np.float32)
+    C[64:80] = 0.0
+    C[100:108] *= np.float32(2.0 ** -124)
+    C[200:208, ::3] *= np.float32(2.0 ** 60)
+    cin = ops.quantize(tt(C), order="c_atb")[0] if packed else layouts.c_layout_atb_values(tt(C, torch.bfloat16))
+    ang = tt(rng.uniform(-np.pi, np.pi, (M, 64)))
+    w = tt(1 + 0.1 * rng.standard_normal((2, 128)))
+    tabs = run_qkv.qkv_tables(torch.cos(ang), torch.sin(ang), w[0] * float(A.C_LOG2), w[1]).reshape(-1)
+    outs = []
+    for general in (False, True):
+        q = torch.full((hq * (M // 64) * 9216,), 3, dtype=torch.uint8, device="cuda")
+        kv = torch.full((hkv * (M // 64) * 2 * 9216,), 3, dtype=torch.uint8, device="cuda")
+        assert run_qkv._stream_form(cin, tabs, q, kv, M, M // 64, hq, hkv)
+        if general:
+            monkeypatch.setattr(run_qkv, "_stream_form", lambda *a: False)
+        run_qkv.qkv_post_run("glue", cin, tabs, q, kv)
+        outs.append((q, kv))
+    assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
