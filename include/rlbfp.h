@@ -220,6 +220,19 @@ int rl_ln_modulate_stream(const uint16_t *x, const void *branch, int32_t br_fmt,
                           int64_t split_row, int32_t norm, uint16_t *x_out, uint8_t *a_packed, int64_t M, int64_t D,
                           void *stream);
 
+/* Row-major values <-> the C-stream element order c_layout_atb(., 128, 128) of (M, D) bf16 values
+ * (redline/npu_layouts.py:31-47), optionally through a column order (the packed weights' channel order,
+ * redline/vlm_run.py:363-371):
+ *   rl_stream_pack:   out[stream(r, c)] = bf16(x[r][perm[c]]) (RNE), rows `rows` .. M - 1 zero;
+ *   rl_stream_unpack: out[r][perm[c]] = x[stream(r, c)].
+ * x / out row major with leading dimension ld, float32 or bf16 (dtype). perm NULL: the identity; otherwise D int64
+ * entries, a permutation of 0 .. D - 1 in device memory, and D <= 8192. M % 512 == 0, D % 1024 == 0; x and out 16-byte
+ * aligned. */
+int rl_stream_pack(const void *x, int32_t dtype, int64_t rows, int64_t ld, const int64_t *perm, int64_t M, int64_t D,
+                   uint16_t *out, void *stream);
+int rl_stream_unpack(const uint16_t *x, const int64_t *perm, int64_t M, int64_t D, void *out, int32_t dtype,
+                     int64_t ld, void *stream);
+
 /* ---- QKV post: the QKV GEMM output -> attention Q / K / V --------------------------------------------------------
  * C (M, 3 * heads * 128) bf16 row major (ldc): per token row the q, k and v columns of `heads` heads of 128 dims.
  * Per head and token row, in fp32:

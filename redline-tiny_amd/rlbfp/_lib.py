@@ -66,6 +66,8 @@ SIGNATURES = {
     "rl_ln_modulate": (ctypes.c_int, [_P, _I64, _P, _I32, _I64, _P, _I64, _I32, _P, _I64, _P, _I32, _P, _I64, _I64,
                                       _I64, _P]),
     "rl_ln_modulate_stream": (ctypes.c_int, [_P, _P, _I32, _P, _I64, _I32, _P, _P, _I64, _I64, _P]),
+    "rl_stream_pack": (ctypes.c_int, [_P, _I32, _I64, _I64, _P, _I64, _I64, _P, _P]),
+    "rl_stream_unpack": (ctypes.c_int, [_P, _P, _I64, _I64, _P, _I32, _I64, _P]),
     "rl_qkv_post": (ctypes.c_int, [_P, _I64, _I64, _I32, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
     "rl_qkv_post_gqa": (ctypes.c_int, [_P, _I64, _I64, _I32, _I32, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
     "rl_qkv_post_stream": (ctypes.c_int, [_P, _I32, _I64, _I32, _I32, _P, _P, _P, _P]),

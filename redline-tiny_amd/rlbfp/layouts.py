@@ -65,15 +65,24 @@ def c_atb_block_index(M, N, device="cuda"):
     return r * (N // 8) + cb
 
 
+def _stream_shape(M, N):
+    """Whether (M, N) bf16 values go to and from the C stream in one kernel (rl_stream_pack / rl_stream_unpack)."""
+    return M >= 512 and M % 512 == 0 and 1024 <= N <= 1 << 24 and N % 1024 == 0
+
+
 def c_layout_atb_values(x):
     """(M, N) device tensor -> its values as a flat C stream, c_layout_atb(x, 128, 128), in x's dtype (e.g. the bf16
     residual stream of redline/run_ln.py:28-30)."""
     M, N = x.shape
+    if _stream_shape(M, N) and x.stride(0) == N and ops.stream_buffer(x, torch.bfloat16, M * N):
+        return ops.stream_pack(x, M, N)
     return x.contiguous().reshape(-1, 8)[c_atb_block_index(M, N, x.device)].reshape(-1)
 
 
 def c_unlayout_atb_values(s, M, N):
     """Flat C stream of values -> (M, N) row major (redline/npu_layouts.py:31-39)."""
+    if _stream_shape(M, N) and ops.stream_buffer(s, torch.bfloat16, M * N):
+        return ops.stream_unpack(s, M, N)
     out = torch.empty((M * N // 8, 8), dtype=s.dtype, device=s.device)
     out[c_atb_block_index(M, N, s.device)] = s.reshape(-1, 8)
     return out.reshape(M, N)

@@ -345,6 +345,25 @@ def stream_buffer(t, dtype, numel, align=16):
         t.data_ptr() % align == 0
 
 
+def stream_pack(x, M, D, perm=None):
+    """Rows of x (rows <= M, D; float32 or bf16, unit column stride), columns taken in the order perm (int64, a
+    permutation) -> flat bf16 in the C-stream element order of (M, D), missing rows zero (rl_stream_pack)."""
+    out = torch.empty(M * D, dtype=torch.bfloat16, device=x.device)
+    dt = L.RL_DTYPE_BF16 if x.dtype == torch.bfloat16 else L.RL_DTYPE_F32
+    ld = x.stride(0) if x.shape[0] > 1 else D  # the stride of a single row (or none) says nothing
+    L.check(L.lib().rl_stream_pack(_ptr(x), dt, x.shape[0], ld, _ptr(perm), M, D, _ptr(out), _stream(x)))
+    return out
+
+
+def stream_unpack(s, M, D, perm=None, dtype=torch.bfloat16):
+    """The inverse: a flat bf16 C stream -> (M, D) float32 or bf16 with column c of the stream's rows at perm[c]
+    (rl_stream_unpack)."""
+    out = torch.empty((M, D), dtype=dtype, device=s.device)
+    dt = L.RL_DTYPE_BF16 if dtype == torch.bfloat16 else L.RL_DTYPE_F32
+    L.check(L.lib().rl_stream_unpack(_ptr(s), _ptr(perm), M, D, _ptr(out), dt, D, _stream(s)))
+    return out
+
+
 def ln_modulate_stream(x, params, branch, x_out, a_out, M, D, split_row=0, norm="layer"):
     """ln_modulate on the C-stream element order: x, x_out flat bf16, branch None, flat bf16 or a uint8 bfp16 stream in
     that order, a_out the uint8 buffer that receives A in the A layout. See rl_ln_modulate_stream in include/rlbfp.h."""

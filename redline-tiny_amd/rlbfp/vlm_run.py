@@ -131,7 +131,11 @@ class LM:
         l0 = self.layers[0]
         self.d = weights.p_in[l0].numel() // 4
         self.f = weights.w[l0, "up"].numel() // 9 * 8 // self.d // 2
-        self.hp = torch.as_tensor(np.asarray(weights.hp), device=device)
+        hp = np.asarray(weights.hp)
+        self.hp = torch.as_tensor(hp, device=device)
+        # one kernel per direction moves rows between the model's channel order and the residual stream
+        self.hp_kernel = m % 512 == 0 and self.d % 1024 == 0 and self.d <= 8192 and hp.dtype == np.int64 and \
+            np.array_equal(np.sort(hp, axis=None), np.arange(self.d))
         self.w = {k: v for k, v in weights.w.items()}
         d, f, T = self.d, self.f, m // 64
         z = lambda n: torch.zeros(n, dtype=torch.bfloat16, device=device)
@@ -172,10 +176,17 @@ class LM:
 
     def load_x(self, x):
         """x (rows, hidden) in the model's channel order; stored in the packed weights' order (:363-366)."""
-        xp = torch.zeros((self.m, self.d), dtype=torch.float32, device=self.hp.device)
-        x = torch.as_tensor(x, device=self.hp.device).float()
-        xp[:x.shape[0]] = x
-        self.x[0] = layouts.c_layout_atb_values(bf(xp[:, self.hp]).to(torch.bfloat16))
+        x = torch.as_tensor(x, device=self.hp.device)
+        if self.hp_kernel and x.dim() == 2 and x.shape[0] <= self.m and x.shape[1] == self.d:
+            x = (x if x.dtype == torch.bfloat16 else x.float()).contiguous()
+            if x.data_ptr() % 16:
+                x = x.clone()
+            self.x[0] = ops.stream_pack(x, self.m, self.d, perm=self.hp)
+        else:
+            xp = torch.zeros((self.m, self.d), dtype=torch.float32, device=self.hp.device)
+            x = x.float()
+            xp[:x.shape[0]] = x
+            self.x[0] = layouts.c_layout_atb_values(bf(xp[:, self.hp]).to(torch.bfloat16))
         self.cur, self.br, self.br16 = 0, self.br_zero, False
 
     def unperm(self, xp):
@@ -215,4 +226,6 @@ class LM:
         """The residual stream after the last layer (x2 + down), via one more rms pass (its A output unused)."""
         x0, x1 = self.x[self.cur], self.x[(self.cur + 1) % 3]
         self._rms(x0, self.br, self.br16, self.wts.p_in[last_i], x1, self.a1)
+        if self.hp_kernel:
+            return ops.stream_unpack(x1, self.m, self.d, perm=self.hp, dtype=torch.float32)
         return self.unperm(layouts.c_unlayout_atb_values(x1, self.m, self.d).float())

@@ -282,3 +282,14 @@ def test_qkv_stream_rejects_before_any_gpu_call():
     assert f(16, 1, 512, 0, 4, 16, 16, 16, None) == L.RL_ERR_SHAPE
     assert f(16, 1, 512, 8, 8, 16, None, 16, None) == L.RL_ERR_NULL
     assert f(16, 1, 512, 8, 8, 8, 16, 16, None) == L.RL_ERR_ALIGN
+
+
+def test_stream_pack_rejects_before_any_gpu_call():
+    f, g = L.lib().rl_stream_pack, L.lib().rl_stream_unpack
+    assert f(16, 0, 100, 1024, None, 500, 1024, 16, None) == L.RL_ERR_SHAPE
+    assert f(16, 0, 100, 9216, 16, 512, 9216, 16, None) == L.RL_ERR_SHAPE   # a permutation of more than 8192 columns
+    assert f(16, 0, 513, 1024, None, 512, 1024, 16, None) == L.RL_ERR_SHAPE
+    assert f(16, 2, 100, 1024, None, 512, 1024, 16, None) == L.RL_ERR_ARG
+    assert f(16, 0, 100, 1020, None, 512, 1024, 16, None) == L.RL_ERR_ALIGN
+    assert f(None, 0, 100, 1024, None, 512, 1024, 16, None) == L.RL_ERR_NULL
+    assert g(16, None, 512, 1000, 16, 0, 1024, None) == L.RL_ERR_SHAPE and g(8, None, 512, 1024, 16, 0, 1024, None) == L.RL_ERR_ALIGN

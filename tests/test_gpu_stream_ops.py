@@ -205,3 +205,27 @@ def test_qkv_stream(dev, monkeypatch, M, hq, hkv, packed):
         run_qkv.qkv_post_run("glue", cin, tabs, q, kv)
         outs.append((q, kv))
     assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])
+
+
+@pytest.mark.parametrize("M,D,rows,dtype", [(512, 1024, 512, torch.float32), (1024, 3072, 777, torch.bfloat16),
+                                            (512, 8192, 1, torch.float32), (512, 2048, 0, torch.bfloat16)])
+def test_stream_pack(dev, M, D, rows, dtype):
+    """Both directions, with and without a column order, short inputs padded with zero rows: the exact values."""
+    rng = np.random.default_rng(M + rows)
+    x = rng.standard_normal((rows, D)).astype(np.float32)
+    perm = rng.permutation(D)
+    xb = np.zeros((M, D), np.float32)
+    xb[:rows] = F.bf16_round(x) if rows else x
+    for p in (None, perm):
+        pt = None if p is None else tt(p, torch.int64)
+        s = ops.stream_pack(tt(x, dtype), M, D, perm=pt)
+        want = F.c_layout_atb(xb if p is None else np.ascontiguousarray(xb[:, p]))
+        np.testing.assert_array_equal(s.float().cpu().numpy(), want)
+        for dt in (torch.float32, torch.bfloat16):
+            back = ops.stream_unpack(s, M, D, perm=pt, dtype=dt)
+            assert back.dtype == dt
+            np.testing.assert_array_equal(back.float().cpu().numpy(), xb)
+    b = layouts.c_layout_atb_values(tt(xb, torch.bfloat16))
+    np.testing.assert_array_equal(b.float().cpu().numpy(), F.c_layout_atb(xb))
+    assert torch.equal(b.float(), layouts.c_layout_atb_values(tt(xb)))
+    assert torch.equal(layouts.c_unlayout_atb_values(b, M, D).float(), layouts.c_unlayout_atb_values(b.float(), M, D))
