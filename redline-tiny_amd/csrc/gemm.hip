@@ -20,6 +20,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "rlbfp.h"
@@ -1234,6 +1235,377 @@ __global__ __launch_bounds__(kW4Threads, 1) void gemm4w_kernel(const GemmArgs<G>
   }
 }
 
+// ---- few rows, few K steps: B decoded straight from memory into MFMA operands ---------------------------------------
+//
+// For M <= 64 and a short enough K (skinny_fits) the tiles above do their work for 256 rows, and a split launch spends
+// most of its time on the partial sums and the second launch. Here a wave owns CG 16-column groups and all rows (MF
+// 16-row fragments). Lane l's B operand of a 16-column x 32-K fragment is block l of 64 consecutive blocks of the b_layout
+// stream (K block l / 16, column l % 16), so the wave loads 576 contiguous bytes as 12-byte windows and decodes them in
+// registers: no LDS tile, no barrier in the loop. The A operand is 16 bytes of row l % 16 per fragment, read through L1 /
+// L2 (A is small and shared by every workgroup). Both come through a ring of P steps in registers. The 8 waves are KS
+// contiguous pieces of K x 8 / KS column sets; the pieces' sums are added in piece order through LDS, so it serves calls
+// that allow a K split. Then bias, activation, gate / residual and rounding as in the other kernels.
+// Measured, weights cold, one launch against the split launch and its reduce, us per call: 4096 x 4096, 1 / 16 rows 19.5 ->
+// 7.4 and 19.6 -> 10.2; K = 3072, 24576 columns, 8 rows 31.6 -> 20.4; 2048 x 2048, 8 rows 15.9 -> 5.3.
+constexpr int kSkThreads = 512;
+template <int MF, int CG>
+constexpr int sk_ring() {
+  if (CG == 1) return MF <= 2 ? 6 : 4;
+  if (CG == 2) return MF <= 2 ? 4 : 3;
+  return MF <= 2 ? 3 : 2;
+}
+
+template <int MF, int CG, int KS>
+__global__ __launch_bounds__(kSkThreads, 2) void gemm_skinny_kernel(const GemmDesc d) {
+  constexpr int NCW = 8 / KS, P = sk_ring<MF, CG>(), kFrags = MF * CG;
+  typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
+  __shared__ __attribute__((aligned(16))) f32x4 lds[8 * kFrags * 64];
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kw = wave % KS, cw = wave / KS;
+  const bool swiglu = d.act == RL_ACT_SWIGLU;
+  const int KT = d.K / BK;
+  const int ngroups = d.N / (16 * CG);
+  // column group c of the wave's set: 16-column band sbc of 128-column tile nt; SwiGLU sets hold gate bands and the proj
+  // bands 4 further on
+  constexpr int kPer = 8 / CG;
+  auto band = [&](int g, int c) {
+    const int i = g % kPer;
+    return swiglu ? (CG / 2) * i + c % (CG > 1 ? CG / 2 : 1) + (c >= CG / 2 ? 4 : 0) : CG * i + c;
+  };
+  const int grp = min((int)blockIdx.x * NCW + cw, ngroups - 1);
+  const int k0 = kw * KT / KS, n = (kw + 1) * KT / KS - k0;
+
+  const __amdgpu_buffer_rsrc_t brs =
+      __builtin_amdgcn_make_buffer_rsrc((void*)d.B, (short)0, (int)((int64_t)d.K * d.N / 8 * 9), 0x00020000);
+  const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)d.A, (short)0, (int)(((int64_t)d.M - 1) * d.lda * 2 + (int64_t)d.K * 2), 0x00020000);
+  const uint32_t vb = (uint32_t)(9 * lane & ~3);
+  const uint32_t bs = (uint32_t)(lane & 3);  // (9 * lane) % 4
+  const uint32_t va = (uint32_t)((int64_t)l16 * d.lda * 2 + lg * 16);
+  const uint32_t row16 = (uint32_t)(16 * d.lda * 2);
+
+  u32x3 rb[P][CG][2];
+  u32x4 ra[P][MF][2];
+  auto load = [&](int p, int s) {
+    const int k = min(k0 + s, KT - 1);
+#pragma unroll
+    for (int c = 0; c < CG; c++)
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+        rb[p][c][h] = __builtin_bit_cast(u32x3, __builtin_amdgcn_raw_buffer_load_b96(
+            brs, vb, (((grp / kPer) * KT + k) * 8 + band(grp, c)) * 1152 + 576 * h, kLoadStream));
+#pragma unroll
+    for (int mf = 0; mf < MF; mf++)
+#pragma unroll
+      for (int h = 0; h < 2; h++)
+        ra[p][mf][h] = __builtin_bit_cast(
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(ars, va + mf * row16, k * (2 * BK) + 64 * h, 0));
+  };
+  f32x4 acc[MF][CG];
+#pragma unroll
+  for (int mf = 0; mf < MF; mf++)
+#pragma unroll
+    for (int c = 0; c < CG; c++) acc[mf][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto compute = [&](int p) {
+#pragma unroll
+    for (int h = 0; h < 2; h++)
+#pragma unroll
+      for (int c = 0; c < CG; c++) {
+        const bf16x8 b = decode_window(rb[p][c][h].x, rb[p][c][h].y, rb[p][c][h].z, bs);
+#pragma unroll
+        for (int mf = 0; mf < MF; mf++)
+          acc[mf][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ra[p][mf][h]), b, acc[mf][c],
+                                                              0, 0, 0);
+      }
+  };
+#pragma unroll
+  for (int p = 0; p < P; p++) load(p, p);
+  int s = 0;
+  for (; s + P <= n; s += P) {
+#pragma unroll
+    for (int p = 0; p < P; p++) {
+      compute(p);
+      load(p, s + p + P);  // past the piece: a step that is not used (past K: the last one again)
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+#pragma unroll
+  for (int p = 0; p < P; p++)
+    if (s + p < n) compute(p);
+
+  // every wave's fragments, then their sums over the K pieces in piece order, bias and activation
+#pragma unroll
+  for (int mf = 0; mf < MF; mf++)
+#pragma unroll
+    for (int c = 0; c < CG; c++) lds[(wave * kFrags + mf * CG + c) * 64 + lane] = acc[mf][c];
+  __syncthreads();
+  const int co = swiglu ? CG / 2 : CG;        // output fragments per row fragment
+  const int items = NCW * MF * co * 64;
+  constexpr int kItems = (NCW * kFrags * 64 + kSkThreads - 1) / kSkThreads;
+  f32x4 v[kItems];
+#pragma unroll
+  for (int i = 0; i < kItems; i++) {
+    const int it = tid + kSkThreads * i;
+    if (it < items) {
+      const int f = it >> 6, w = f / (MF * co), mf = (f / co) % MF, c = f % co;
+      auto sum = [&](int cc) {
+        const f32x4* p = lds + (w * KS * kFrags + mf * CG + cc) * 64 + (it & 63);
+        f32x4 t = p[0];
+#pragma unroll
+        for (int k = 1; k < KS; k++) t += p[k * kFrags * 64];
+        return t;
+      };
+      const int g = min((int)blockIdx.x * NCW + w, ngroups - 1);
+      const int col = 128 * (g / kPer) + 16 * band(g, c) + (it & 15);
+      f32x4 x = sum(c);
+      if (d.bias) x += d.bias[col];
+      if (swiglu) {
+        f32x4 u = sum(c + CG / 2);
+        if (d.bias) u += d.bias[col + 64];
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[e] = silu_f(x[e]) * u[e];
+      } else if (d.act == RL_ACT_GELU_TANH) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[e] = gelu_tanh_f(x[e]);
+      }
+      v[i] = x;
+    }
+  }
+  __syncthreads();
+  // row-quad layout: the 4 rows of quad q, staged column c of set w at [(w * 4 MF + q) * W + c]
+  const int W = 16 * co;
+#pragma unroll
+  for (int i = 0; i < kItems; i++) {
+    const int it = tid + kSkThreads * i;
+    if (it < items) {
+      const int f = it >> 6, w = f / (MF * co), mf = (f / co) % MF, c = f % co;
+      lds[(w * 4 * MF + 4 * mf + ((it >> 4) & 3)) * W + 16 * c + (it & 15)] = v[i];
+    }
+  }
+  __syncthreads();
+  const int nout = swiglu ? d.N / 2 : d.N, nblk = W / 8;
+  for (int it = tid; it < NCW * 4 * MF * nblk; it += kSkThreads) {
+    const int w = it / (4 * MF * nblk), q = (it / nblk) % (4 * MF), cb = it % nblk;
+    const int g = (int)blockIdx.x * NCW + w, row0 = 4 * q;
+    if (g >= ngroups || row0 >= d.M) continue;
+    const int col = g * W + 8 * cb;  // a set's output columns are consecutive
+    float x[4][8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      const f32x4 t = lds[(w * 4 * MF + q) * W + 8 * cb + k];
+#pragma unroll
+      for (int i = 0; i < 4; i++) x[i][k] = t[i];
+    }
+    u32x4 o[4];
+    finish_rows4(d, row0, col, nout, x, o);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      if (row0 + i < d.M) *reinterpret_cast<u32x4*>(d.C + (int64_t)(row0 + i) * d.ldc + col) = o[i];
+  }
+}
+
+template <int MF, int CG, int KS>
+static int launch_skinny_v(const GemmDesc& d, void* stream) {
+  const int sets = d.N / (16 * CG), per = 8 / KS;
+  hipLaunchKernelGGL((gemm_skinny_kernel<MF, CG, KS>), dim3((unsigned)((sets + per - 1) / per)), dim3(kSkThreads), 0,
+                     static_cast<hipStream_t>(stream), d);
+  return launch_status("rl_bfp16_gemm");
+}
+template <int CG, int KS>
+static int launch_skinny_mf(const GemmDesc& d, void* stream) {
+  const int mf = (d.M + 15) / 16;
+  if (mf <= 1) return launch_skinny_v<1, CG, KS>(d, stream);
+  if (mf <= 2) return launch_skinny_v<2, CG, KS>(d, stream);
+  if (mf <= 3) return launch_skinny_v<3, CG, KS>(d, stream);
+  return launch_skinny_v<4, CG, KS>(d, stream);
+}
+
+// ---- few rows, many K steps: one 128-column tile per workgroup ------------------------------------------------------
+//
+// For M <= 128 one workgroup holds all rows of a 128-column tile (whole K, or one K piece): 8 waves of one 16-column band
+// each, MF 16-row fragments. A and the raw bytes of B go to LDS by direct loads (1 KB per instruction, whole lines;
+// 12-byte window loads from memory instead cost 16-18% at 64 rows) through a ring of NS stages of two K steps, so that up
+// to NS - 1 stages of the weight stream are in flight per compute unit; each wave decodes its own blocks, once, from
+// 12-byte LDS windows straight into MFMA operands. With two row sets of four waves (half the A reads, every block decoded
+// twice) it took 1.3x as long. The sums run over K in the order of the kernels above: the same bits.
+// Measured against the 4- and 8-wave kernels, weights cold, us per call: K = 4096, 4096 columns, 8 pieces and the reduce
+// launch: 64 rows 23.0 -> 16.3, 77 rows 24.3 -> 17.9, 128 rows 27.0 -> 23.2; whole K 65 -> 33 / 36 / 45. K = 3072, 24576
+// columns: 64 rows 36.6 -> 27.2, 128 rows 42.1 -> 38.2 (whole against the 2-piece launch). A step takes 0.4 us at 16
+// rows and 0.7 at 128: the decode's VALU chains and the LDS operand reads of two waves per SIMD bound it, not memory.
+// A barrier that leaves this wave's vector loads in flight (__syncthreads waits for direct-to-LDS loads): LDS reads are
+// complete, and the caller has waited for the loads that the other waves will read.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+template <int MF>
+__global__ __launch_bounds__(kSkThreads, 2) void gemm_rows_kernel(const GemmDesc d) {
+  constexpr int S = 2, R = 16 * MF;                  // K steps per chunk, rows
+  constexpr int kStepA = R * BK * 2;                // bytes of A per step
+  constexpr int kStage = S * (kStepA + kTileBytes); // a stage: A of the chunk's steps, then the raw B tiles
+  constexpr int NS = 158 * 1024 / kStage < 6 ? 158 * 1024 / kStage : 6;  // stages
+  constexpr int nA = S * R / 8, LA = (nA + 7) / 8;  // A loads (8 rows of one step, 1 KB) per chunk; per wave
+  constexpr int nB = S * 9, LB = (nB + 7) / 8;      // B loads (1 KB of a tile)
+  constexpr int kEp = R * 128 * 4;
+  __shared__ __attribute__((aligned(16))) uint8_t lds[(NS * kStage > kEp ? NS * kStage : kEp) + 1024];
+  uint8_t* const dummy = lds + sizeof(lds) - 1024;  // where the loads that even out the waves' counts go
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, lg = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int KT = d.K / BK, tiles = d.N >> 7;
+  const int pid = xcd_remap(blockIdx.x, gridDim.x);
+  const int piece = pid / tiles, nt = pid - piece * tiles;
+  const int k0 = piece * KT / d.ksplit, n = (piece + 1) * KT / d.ksplit - k0;
+
+  const __amdgpu_buffer_rsrc_t brs =
+      __builtin_amdgcn_make_buffer_rsrc((void*)d.B, (short)0, (int)((int64_t)d.K * d.N / 8 * 9), 0x00020000);
+  const __amdgpu_buffer_rsrc_t ars = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)d.A, (short)0, (int)(((int64_t)d.M - 1) * d.lda * 2 + (int64_t)d.K * 2), 0x00020000);
+  constexpr uint32_t kOut32 = 0x80000000u;  // past every buffer: steps past the piece read zeros
+  // load j of a chunk's A: step s, rows 8 g .. + 7; lane = (row, 16-byte chunk ^ swizzle). a_swz(r) has period 16 in r,
+  // so the lane's offset depends on the parity of g only
+  uint32_t va[2];
+#pragma unroll
+  for (int i = 0; i < 2; i++)
+    va[i] = (uint32_t)((lane >> 3) * (uint32_t)(d.lda * 2) + (((lane & 7) ^ a_swz(8 * i + (lane >> 3))) << 4));
+  const uint32_t row8 = (uint32_t)(8 * d.lda * 2);
+  auto load = [&](int stage, int c) {
+    __builtin_amdgcn_sched_barrier(0);
+    uint8_t* const st = lds + stage * kStage;
+#pragma unroll
+    for (int i = 0; i < LB; i++) {
+      const int j = wave + 8 * i, s = j / 9, q = j - 9 * s, k = S * c + s;
+      const bool on = j < nB && k < n;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          brs, (__attribute__((address_space(3))) void*)(j < nB ? st + S * kStepA + j * 1024 : dummy), 16,
+          on ? 16 * (uint32_t)lane : kOut32, on ? (nt * KT + k0 + k) * kTileBytes + q * 1024 : 0, 0, kLoadStream);
+    }
+#pragma unroll
+    for (int i = 0; i < LA; i++) {
+      const int j = wave + 8 * i, s = j / (R / 8), g = j - s * (R / 8), k = S * c + s;
+      const bool on = j < nA && k < n;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          ars, (__attribute__((address_space(3))) void*)(j < nA ? st + j * 1024 : dummy), 16,
+          on ? va[g & 1] + (uint32_t)g * row8 : kOut32, on ? (k0 + k) * BK * 2 : 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  f32x4 acc[MF];
+#pragma unroll
+  for (int mf = 0; mf < MF; mf++) acc[mf] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint32_t ao0 = l16 * (BK * 2) + ((lg ^ a_swz(l16)) << 4);
+  const uint32_t ao1 = l16 * (BK * 2) + (((4 + lg) ^ a_swz(l16)) << 4);
+  const uint32_t bo = (uint32_t)(wave * 1152 + (9 * lane & ~3));
+  const uint32_t bs = (uint32_t)(lane & 3);  // (9 * lane) % 4
+  // half steps t = 2 s + h; the operands of t + 1 are read while t is multiplied
+  auto compute = [&](const uint8_t* st) {
+    bf16x8 a[2][MF];
+    uint32_t w[2][3];
+    auto read = [&](int t) {
+      const uint8_t* as = st + (t >> 1) * kStepA + (t & 1 ? ao1 : ao0);
+      const uint8_t* bp = st + S * kStepA + (t >> 1) * kTileBytes + (t & 1) * 576 + bo;
+#pragma unroll
+      for (int i = 0; i < 3; i++) w[t & 1][i] = reinterpret_cast<const uint32_t*>(bp)[i];
+#pragma unroll
+      for (int mf = 0; mf < MF; mf++) a[t & 1][mf] = *reinterpret_cast<const bf16x8*>(as + mf * 16 * (BK * 2));
+    };
+    read(0);
+#pragma unroll
+    for (int t = 0; t < 2 * S; t++) {
+      if (t + 1 < 2 * S) read(t + 1);
+      const bf16x8 b = decode_window(w[t & 1][0], w[t & 1][1], w[t & 1][2], bs);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int mf = 0; mf < MF; mf++)
+        acc[mf] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[t & 1][mf], b, acc[mf], 0, 0, 0);
+    }
+  };
+  // ring of NS stages: chunks c + 1 .. c + NS - 2 are in flight while chunk c is waited for; its stage was last read
+  // before the barrier that the refill follows
+  const int nc = (n + S - 1) / S;
+#pragma unroll
+  for (int i = 0; i < NS - 1; i++) load(i, i);
+  int stage = 0, fill = NS - 1;
+  for (int c = 0; c < nc; c++) {
+    wait_vm<(NS - 2) * (LA + LB)>();
+    lds_barrier();
+    load(fill, c + NS - 1);
+    compute(lds + stage * kStage);
+    stage = stage + 1 == NS ? 0 : stage + 1;
+    fill = fill + 1 == NS ? 0 : fill + 1;
+  }
+  wait_vm<0>();
+  __syncthreads();  // no load into the stages is left before they are reused or the workgroup ends
+  const int n0 = 128 * nt;
+  if (d.ksplit > 1) {
+    float* part = d.part + (int64_t)piece * d.M * d.N + n0 + 16 * wave + l16;
+#pragma unroll
+    for (int mf = 0; mf < MF; mf++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int row = 16 * mf + 4 * lg + i;
+        if (row < d.M) part[(int64_t)row * d.N] = acc[mf][i];
+      }
+    return;
+  }
+  // whole K: the tile in the row-quad layout, then 4 rows x 8 columns per thread
+  f32x4* ep = reinterpret_cast<f32x4*>(lds);
+#pragma unroll
+  for (int mf = 0; mf < MF; mf++) ep[(4 * mf + lg) * 128 + ep_slot(16 * wave + l16)] = acc[mf];
+  __syncthreads();
+  const bool swiglu = d.act == RL_ACT_SWIGLU;
+  const int nout = swiglu ? d.N / 2 : d.N, nblk = swiglu ? 8 : 16;
+  for (int it = tid; it < (R / 4) * nblk; it += kSkThreads) {
+    const int q = it / nblk, cb = it % nblk, row0 = 4 * q;
+    if (row0 >= d.M) continue;
+    float v[4][8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+      f32x4 x = ep[q * 128 + ep_slot(8 * cb + k)];
+      if (d.bias) x += d.bias[n0 + 8 * cb + k];
+      if (swiglu) {
+        f32x4 u = ep[q * 128 + ep_slot(64 + 8 * cb + k)];
+        if (d.bias) u += d.bias[n0 + 64 + 8 * cb + k];
+#pragma unroll
+        for (int i = 0; i < 4; i++) x[i] = silu_f(x[i]) * u[i];
+      } else if (d.act == RL_ACT_GELU_TANH) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) x[i] = gelu_tanh_f(x[i]);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; i++) v[i][k] = x[i];
+    }
+    const int col = (swiglu ? n0 / 2 : n0) + 8 * cb;
+    u32x4 o[4];
+    finish_rows4(d, row0, col, nout, v, o);
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      if (row0 + i < d.M) *reinterpret_cast<u32x4*>(d.C + (int64_t)(row0 + i) * d.ldc + col) = o[i];
+  }
+}
+
+template <int MF>
+static int launch_rows_v(const GemmDesc& d, void* stream) {
+  hipLaunchKernelGGL(gemm_rows_kernel<MF>, dim3((unsigned)((d.N >> 7) * d.ksplit)), dim3(kSkThreads), 0,
+                     static_cast<hipStream_t>(stream), d);
+  return launch_status("rl_bfp16_gemm");
+}
+constexpr int kRowsMax = 128;
+static int launch_rows(const GemmDesc& d, void* stream) {
+  switch ((d.M + 15) / 16) {
+    case 1: return launch_rows_v<1>(d, stream);
+    case 2: return launch_rows_v<2>(d, stream);
+    case 3: return launch_rows_v<3>(d, stream);
+    case 4: return launch_rows_v<4>(d, stream);
+    case 5: return launch_rows_v<5>(d, stream);
+    case 6: return launch_rows_v<6>(d, stream);
+    case 7: return launch_rows_v<7>(d, stream);
+    default: return launch_rows_v<8>(d, stream);
+  }
+}
+
 template <int G>
 static int fill_desc(GemmDesc& g, const void* A, int64_t lda, const uint8_t* B, uint16_t* C, int64_t ldc, int64_t M,
                      int64_t N, int64_t K, const rl_epilogue* ep, int32_t a_fmt, int tile_start) {
@@ -1311,6 +1683,22 @@ static Plan8 plan8(int64_t M, int64_t N, int cus) {
     }
   }
   return best;
+}
+
+// gemm_skinny_kernel's range: its time grows with rows x K (every workgroup reads its K pieces of A through L1), the
+// split launch's hardly does. The line is where they cross: measured at 3072-4096 columns, 16 rows 10.2 against 13.0 us
+// at K = 4096 and 22 against 18 at 12288; 33 rows 15.1 against 14.5 at 4096 and 10.5 against 10.9 at 2048; 64 rows 15.7
+// against 11.8 at 2048 and 8.8 against 9.7 at K = 1024.
+static bool skinny_fits(int64_t M, int64_t K) { return M <= 64 && (M + 15) / 16 * 16 * K <= (1 << 17); }
+
+// Column sets: one round of workgroups with the narrowest set (16 columns of all 8 K pieces per workgroup up to 4096
+// columns), wider sets for wider outputs (24576 columns, 16 rows: 22.5 us with 64-column sets x 4 pieces, 26 with 32 x 8).
+static int launch_skinny(const GemmDesc& d, int cus, void* stream) {
+  const int groups = d.N / 16;
+  if (groups <= cus && d.act != RL_ACT_SWIGLU) return launch_skinny_mf<1, 8>(d, stream);
+  if (groups <= 2 * cus) return launch_skinny_mf<2, 8>(d, stream);
+  if (groups <= 4 * cus) return launch_skinny_mf<4, 8>(d, stream);
+  return launch_skinny_mf<4, 4>(d, stream);
 }
 
 // ---- whole-K plan over both kernels -----------------------------------------------------------------------------
@@ -1539,8 +1927,12 @@ static GemmDesc rows_from(const GemmDesc& g, int64_t R) {
   return t;
 }
 
+// Whole-K launches of at most 128 rows into a row-major C (second launches too): gemm_rows_kernel
+static bool rows_serves(const GemmDesc& g) { return g.M <= kRowsMax && !g.pk && !g.c_atb && !kernel_restriction(); }
+
 // One whole-K GEMM (a filled descriptor, bf16 A) as the plan's one or two launches.
 static int launch_planned(const GemmDesc& g, const PlanG& p, void* stream) {
+  if (rows_serves(g)) return launch_rows(g, stream);
   GemmArgs<1> args, tail;
   args.d[0] = g;
   args.n = tail.n = 1;
@@ -1557,6 +1949,7 @@ static int launch_planned(const GemmDesc& g, const PlanG& p, void* stream) {
     s = launch8<1>(args, total, p.mf, stream);
   }
   if (s || !p.split) return s;
+  if (rows_serves(tail.d[0])) return launch_rows(tail.d[0], stream);
   if (p.tail_w4) {
     set_tiles4w(tail, p.mf_tail, total);
     return launch4w<1>(tail, total, p.mf_tail, stream);
@@ -1667,9 +2060,19 @@ int rl_bfp16_gemm_ws(const void* A, int32_t a_fmt, int64_t lda, const uint8_t* B
       if (sp.ws_bytes > workspace_bytes)
         return fail(RL_ERR_WORKSPACE, "workspace %lld bytes, this shape needs %lld (rl_bfp16_gemm_workspace_bytes)",
                     (long long)workspace_bytes, (long long)sp.ws_bytes);
-      args.d[0].ksplit = sp.ks;
       args.d[0].part = static_cast<float*>(workspace);
-      if (sp.w4) {
+      args.d[0].ksplit = sp.ks;
+      if (M <= kRowsMax && !kernel_restriction()) {
+        // few rows: at most the plan's pieces (its partial sums fit the workspace), in one round of workgroups
+        const bool rowmajor = !args.d[0].pk && !args.d[0].c_atb;
+        if (rowmajor && skinny_fits(M, K)) {
+          args.d[0].ksplit = 1;
+          return launch_skinny(args.d[0], device_cus(), stream);
+        }
+        const int fit = std::max(1, device_cus() / (int)(N / 128));
+        args.d[0].ksplit = rowmajor ? std::min(sp.ks, fit) : std::max(2, std::min(sp.ks, fit));
+        if ((s = launch_rows(args.d[0], stream)) || args.d[0].ksplit == 1) return s;
+      } else if (sp.w4) {
         set_tiles4w(args, sp.mf, total);
         if ((s = launch4w<1>(args, total, sp.mf, stream))) return s;
       } else {
