@@ -367,6 +367,7 @@ __global__ __launch_bounds__(W * 64, 8 / W) void attn_kernel(AttnArgs a) {
     float alpha[2];
     bool rebased[2];
     scores(0);
+    __syncthreads();                   // every wave has read K(0): iteration 0 stores K(2) into its buffer
     softmax(kb0, Pb, alpha, rebased);  // O is still 0: no rescale
     // Every load and store below is unconditional: past the last block they repeat block kb1 - 1 into a buffer that is
     // not read again, which keeps the loop free of branches around memory operations. The loop runs two blocks per

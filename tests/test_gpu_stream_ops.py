@@ -229,3 +229,18 @@ def test_stream_pack(dev, M, D, rows, dtype):
     np.testing.assert_array_equal(b.float().cpu().numpy(), F.c_layout_atb(xb))
     assert torch.equal(b.float(), layouts.c_layout_atb_values(tt(xb)))
     assert torch.equal(layouts.c_unlayout_atb_values(b, M, D).float(), layouts.c_unlayout_atb_values(b.float(), M, D))
+
+
+@pytest.mark.parametrize("H,N", [(24, 4352), (24, 1152)])
+def test_attention_deterministic_on_cold_caches(dev, H, N):
+    """The same bits on every launch, with K, V and Q pushed out of the caches before each: the waves of a workgroup then
+    run far apart, and a key block that is overwritten before all of them have read it shows."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    q, k, v = (torch.randn((H, N, 128), generator=g, device="cuda").bfloat16() for _ in range(3))
+    vt = v.transpose(1, 2).contiguous()
+    q = q * float(A.C_LOG2)
+    big = torch.zeros(1 << 28, dtype=torch.uint8, device="cuda")
+    ref = ops.attention(q, k, vt, split=False)
+    for i in range(12):
+        big.add_(1)
+        assert torch.equal(ops.attention(q, k, vt, split=False), ref), i
