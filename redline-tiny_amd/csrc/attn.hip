@@ -369,24 +369,74 @@ __global__ __launch_bounds__(W * 64, 8 / W) void attn_kernel(AttnArgs a) {
     scores(0);
     __syncthreads();                   // every wave has read K(0): iteration 0 stores K(2) into its buffer
     softmax(kb0, Pb, alpha, rebased);  // O is still 0: no rescale
+    // Scores of block j + 1 and P(j) V(j): 32 operand reads, each feeding two MFMAs, kept kAhead reads ahead of their
+    // products (left to the compiler each read stood right before its MFMAs and its latency in full), and ordered so that
+    // consecutive MFMAs accumulate into different registers. kAhead is the most that compiles without spills; the 4-wave
+    // kernel has no registers for it (twice the staging registers per thread) and leaves the order to the compiler.
+    // 24 heads x 4352 x 4352: 226 -> 219 us, 32 x 4096 x 8256: 469 -> 454 us (1220 TFLOP/s), same bits. The two waves of
+    // a SIMD taking turns (one in its MFMAs, one in its softmax, changing over at a second barrier per block) gave 235 and
+    // 493 us with the same reads: the matrix pipes are limited by the board's power here, not by the waves' phases.
+    auto products = [&]<int P>() {
+      const uint8_t* sk = kbuf + (1 - P) * kAtK;
+      const uint8_t* sv = vbuf + P * kAtK;
+      constexpr int kAhead = LIM ? 5 : 7;
+      bf16x8 fr[kAhead];
+      auto rd = [&](int i) {
+        if (i < 16) {
+          const int st = i >> 2, key = 16 * (i & 3) + l16;
+          return *reinterpret_cast<const bf16x8*>(sk + key * 256 + (((4 * st + lg) ^ l16) << 4));
+        }
+        const int c = (i - 16) >> 3, dg = i & 7;
+        return *reinterpret_cast<const bf16x8*>(sv + (16 * dg + l16) * 128 + (((4 * c + lg) ^ vswz(l16)) << 4));
+      };
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int i = 0; i < kAhead; i++) fr[i] = rd(i);
+#pragma unroll
+      for (int i = 0; i < 32; i++) {
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+          if (i < 16)
+            S[s][i & 3] = mfma16(fr[i % kAhead], qB[s][i >> 2], i < 4 ? nb4[s] : S[s][i & 3]);
+          else
+            O[s][i & 7] = mfma16(fr[i % kAhead], __builtin_bit_cast(bf16x8, Pb[s][(i - 16) >> 3]), O[s][i & 7]);
+        }
+        if (i + kAhead < 32) fr[i % kAhead] = rd(i + kAhead);
+      }
+      constexpr int kMfma = 0x008, kDsRead = 0x100;
+      __builtin_amdgcn_sched_group_barrier(kDsRead, kAhead, 0);
+#pragma unroll
+      for (int i = 0; i < 32; i++) {
+        __builtin_amdgcn_sched_group_barrier(kMfma, 2, 0);
+        if (i + kAhead < 32) __builtin_amdgcn_sched_group_barrier(kDsRead, 1, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
     // Every load and store below is unconditional: past the last block they repeat block kb1 - 1 into a buffer that is
     // not read again, which keeps the loop free of branches around memory operations. The loop runs two blocks per
     // trip, so each buffer index is a constant (an immediate LDS offset, no address arithmetic per block).
     auto iter = [&]<int P>(int j) {  // P = j % 2
       load_v(kb0 + j + 1);
       load_k(kb0 + min(j + 2, nb - 1));
-      scores(1 - P);
-      pv(P, Pb);
       u32x4 Pn[2][2];
-      softmax(kb0 + j + 1, Pn, alpha, rebased);
+      if constexpr (W == 8) {
+        products.template operator()<P>();
+        softmax(kb0 + j + 1, Pb, alpha, rebased);
+      } else {
+        scores(1 - P);
+        pv(P, Pb);
+        softmax(kb0 + j + 1, Pn, alpha, rebased);
+      }
 #pragma unroll
       for (int s = 0; s < 2; s++) {
         if (rebased[s]) {  // O has P(j) V(j) now; a rebase at block j + 1 applies to all of it
 #pragma unroll
           for (int dg = 0; dg < 8; dg++) O[s][dg] *= alpha[s];
         }
+        if constexpr (W != 8) {
 #pragma unroll
-        for (int c = 0; c < 2; c++) Pb[s][c] = Pn[s][c];
+          for (int c = 0; c < 2; c++) Pb[s][c] = Pn[s][c];
+        }
       }
       store_v(1 - P);  // V buffer (j + 1) % 2 held V(j - 1), read in iteration j - 1
       store_k(P);      // K buffer j % 2 held K(j), read in iteration j - 1
