@@ -672,8 +672,26 @@ static AttnPlan attn_plan(int32_t heads, int64_t nq, int64_t nk, int cus) {
   const int64_t rem = p.ntask % R;
   if (rem == 0 || rem * 5 > R * 4) return p;
   const int64_t tail = rem * nblk;
-  const int64_t per = std::max<int64_t>(4, (tail + R - 1) / R);
+  int64_t per = std::max<int64_t>(4, (tail + R - 1) / R);
   if (per >= nblk || (int64_t)p.ntask * nblk > INT32_MAX) return p;
+  if (p.ntask < R) {
+    // every task fits at once: the split shortens the chain of key blocks but pays for its partial sums and the second
+    // launch. Model in us, from launches of 1 to 32 heads x 256 to 4352 tokens: a key block takes 1.62 (8 waves), 1.36 (4
+    // waves, one workgroup per CU) or 2.16 (two), the merge 4.5 + 0.42 per MB of partials. Whole against split, measured:
+    // 24 x 1152^2 32.7 against 43.9, 32 x 1152 x 1088 44.7 against 53.3, 24 x 512^2 21.6 against 24.4, 8 x 2176^2 53.6
+    // against 44.9 (split), 4 x 4352^2 119 against 61 (split).
+    auto block_us = [&](int64_t nwg) { return p.w == 8 ? 1.62 : nwg <= cus ? 1.36 : 2.16; };
+    double best = (double)nblk * block_us(p.ntask);
+    int64_t best_per = nblk;
+    for (int64_t x = per; x < nblk; x++) {
+      const int64_t nr = (tail + x - 1) / x;  // ranges; a range boundary inside a task adds a piece to it
+      const double mb = (double)(p.ntask + nr) * part_floats(qt) * 4e-6;
+      const double c = (double)x * block_us(nr) + 4.5 + 0.42 * mb;
+      if (c < best) { best = c; best_per = x; }
+    }
+    if (best_per >= nblk) return p;
+    per = best_per;  // at least the ranges' minimum above: never more pieces or workspace than that
+  }
   p.nfull = (int32_t)(p.ntask - rem);
   p.per = (int32_t)per;
   p.mp = (int32_t)((nblk + per - 1) / per + 1);

@@ -293,3 +293,18 @@ def test_stream_pack_rejects_before_any_gpu_call():
     assert f(16, 0, 100, 1020, None, 512, 1024, 16, None) == L.RL_ERR_ALIGN
     assert f(None, 0, 100, 1024, None, 512, 1024, 16, None) == L.RL_ERR_NULL
     assert g(16, None, 512, 1000, 16, 0, 1024, None) == L.RL_ERR_SHAPE and g(8, None, 512, 1024, 16, 0, 1024, None) == L.RL_ERR_ALIGN
+
+
+def test_attention_split_plan():
+    """The split's workspace: none where whole tasks are quicker than partial sums and a merge, some where a few tasks
+    leave most of the GPU idle, and within one piece per 4 key blocks (256 compute units when no device is present)."""
+    f = L.lib().rl_attention_workspace_bytes
+    part = lambda w: (32 * w * 128 + 2 * 32 * w) * 4
+    for heads, nq, nk, split in ((24, 1152, 1152, False), (32, 1152, 1088, False), (24, 512, 512, False),
+                                 (8, 2176, 2176, True), (4, 4352, 4352, True), (1, 4352, 4352, True),
+                                 (24, 4352, 4352, True), (24, 256, 256, False), (32, 4096, 8256, False)):
+        n = f(heads, nq, nk)
+        assert (n > 0) == split, (heads, nq, nk, n)
+        w = 8 if nq % 256 == 0 else 4
+        tasks = heads * nq // (32 * w)
+        assert n <= tasks * (-(-(nk // 64) // 4) + 1) * part(w)
