@@ -29,6 +29,14 @@ constexpr int kBlockBytes = 9;
 // the bit measured slower there (quantize 13.2 -> 13.8 us, LN 22.8 -> 24.2 us).
 constexpr int kLoadStream = 2;
 
+// A 16-byte store with the non-temporal bit: for outputs that the next kernels do not read (the residual stream x' comes
+// back only after three GEMMs and attention have passed through the caches). Kept out of the caches they do not push out
+// what is being read: residual + norm at 4352 x 3072 21.4 -> 19.4 us, on streams at 4096 x 4096 28.1 -> 22.9 us. A
+// GEMM's A operand, written by the pass before it, keeps the default policy.
+__device__ __forceinline__ void store_stream(void* p, u32x4 v) {
+  __builtin_nontemporal_store(v, static_cast<u32x4*>(p));
+}
+
 // ---- exact encode: integer arithmetic on the float32 bit pattern -----------------------------------------------
 
 // Largest exponent field of 8 float32 bit patterns.
