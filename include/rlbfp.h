@@ -126,7 +126,8 @@ int rl_bfp16_gemm(const void *A, int32_t a_fmt, int64_t lda, const uint8_t *B_pa
  *   - a GEMM whose output tiles fill few compute units (small M, deep K: the text encoder's down projection at
  *     M = 512, K = 12288) may split K into pieces that run side by side. Each piece writes fp32 partial sums to the
  *     workspace; a second launch adds them in piece order and applies the epilogue as above (results differ from
- *     the whole-K sums by fp32 rounding only);
+ *     the whole-K sums by fp32 rounding only). At most 64 rows of a short K run the pieces and their sum in one launch,
+ *     which leaves the workspace untouched;
  *   - an A in any format other than RL_A_BF16 (the NPU's packed A layout above all: every GEMM of
  *     redline/forward.py passes A that way, :32, :245) is first staged as bf16 in the workspace (its exact bfp16
  *     values, one HBM-bound pass: 9/8 + 2 bytes per value), and the product then runs on the RL_A_BF16 kernel with

@@ -275,9 +275,9 @@ __global__ __launch_bounds__(W * 64, 8 / W) void attn_kernel(AttnArgs a) {
       }
     };
 
-    // online softmax (base 2) of key block b (absolute index): P^T -> Pb (bf16), row sums into lsum; alpha[s] is the factor O must take
-    // (after its P V products of the previous block) when the running max was rebased, rebased[s] whether any lane of
-    // the set did. The four lanes l16, l16 + 16, + 32, + 48 hold a query's 64 keys.
+    // online softmax (base 2) of key block b (absolute index): P^T -> Pb (bf16), row sums into lsum; alpha[s] is the factor
+    // O must take (after its P V products of the previous block) when the running max was rebased, rebased[s] whether any
+    // lane of the set did. The four lanes l16, l16 + 16, + 32, + 48 hold a query's 64 keys.
     auto softmax = [&](int b, u32x4 (&Pb)[2][2], float (&alpha)[2], bool (&rebased)[2]) {
       const bool full = (b + 1) * kAtKB <= vis;
 #pragma unroll

@@ -309,9 +309,10 @@ static int launch_upto(int nb, const LnArgs& a, hipStream_t st) {
 // share their cache lines; xcd_remap puts them on one XCD. A row's values are spread over the lanes of equal rib of
 // all 8 waves, so the mean and the variance take a wave reduction, an LDS exchange and a barrier each.
 // HBM-bound: 2 + 9/8 (or 2) bytes read and 2 + 9/8 written per value, once. 4096 x 4096 with a packed branch (105 MB)
-// replaces index-tensor permutations of x and x', a dequantize pass, the row-major kernel and a copy (1063 us);
-// it takes 22.9 us (4.6 TB/s; 28.1 with cached stores of x'). All of a row's loads are issued before the first use; 8 rows x D values stay in registers
-// as bf16 pairs (32 VGPRs at D = 4096: the 512 workgroups of 4096 rows are all resident, 2 per CU).
+// replaces index-tensor permutations of x and x', a dequantize pass, the row-major kernel and a copy (1063 us); it takes
+// 22.9 us (4.6 TB/s; 28.1 with cached stores of x'). All of a row's loads are issued before the first use; 8 rows x D
+// values stay in registers as bf16 pairs (32 VGPRs at D = 4096: the 512 workgroups of 4096 rows are all resident, 2 per
+// CU).
 constexpr int kLsThreads = 512, kLsRows = 8;
 
 struct LnStreamArgs {

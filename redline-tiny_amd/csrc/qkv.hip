@@ -301,8 +301,9 @@ __global__ __launch_bounds__(kQkvThreads) void qkv_stream_kernel(QkvStreamArgs a
 // dword-aligned run (two 16-byte loads and one 4-byte load) holding rows r .. r + 3 (V: dims) of one 8-value block
 // column, so each store instruction of a wave fills whole 256-byte (V: 128-byte) rows. HBM-bound: 9/8 bytes read and 2
 // written per value; it replaces index-tensor gathers, float32 copies and concatenations of every operand (32 heads, 4096
-// queries, 8256 keys, with the packed O below: the whole attention step 4960 -> 1155 us). Decoding inside the attention kernel instead would cost every workgroup of a head the same ~100
-// VALU instructions per wave and key block, beside 112 of the softmax.
+// queries, 8256 keys: 43 us; with the QKV post's stream form and packed O, the attention step with its two GEMMs took
+// 4950 us and takes 1005). Decoding inside the attention kernel instead would cost every workgroup of a head the same
+// ~100 VALU instructions per wave and key block, beside 112 of the softmax.
 struct TilesArgs {
   const uint8_t* q_tiles;
   int32_t hq, q_all, q_t0, q_n, q_out;  // heads, tiles per head in the source, first tile, tiles there, tiles written
