@@ -1427,8 +1427,9 @@ static int launch_skinny_mf(const GemmDesc& d, void* stream) {
 // each, MF 16-row fragments. A and the raw bytes of B go to LDS by direct loads (1 KB per instruction, whole lines;
 // 12-byte window loads from memory instead: 17.1 against 16.3 us at 64 rows, 22.4 against 17.9 at 77, 4096 x 4096 in 8
 // pieces) through a ring of NS stages of two K steps, so that up to NS - 1 stages of the weight stream are in flight per
-// compute unit; each wave decodes its own blocks, once, from 12-byte LDS windows straight into MFMA operands. With two row sets of four waves (half the A reads, every block decoded
-// twice) it took 1.3x as long. The sums run over K in the order of the kernels above: the same bits.
+// compute unit; each wave decodes its own blocks, once, from 12-byte LDS windows straight into MFMA operands. With two
+// row sets of four waves (half the A reads, every block decoded twice) it took 1.3x as long. The sums run over K in the
+// order of the kernels above: the same bits.
 // Measured against the 4- and 8-wave kernels, weights cold, us per call: K = 4096, 4096 columns, 8 pieces and the reduce
 // launch: 64 rows 23.0 -> 16.3, 77 rows 24.3 -> 17.9, 128 rows 27.0 -> 23.2; whole K 65 -> 33 / 36 / 45. K = 3072, 24576
 // columns: 64 rows 36.6 -> 27.2, 128 rows 42.1 -> 38.2 (whole against the 2-piece launch). A step takes 0.4 us at 16

@@ -338,10 +338,23 @@ def overlaps(a, b):
         b.data_ptr() < a.data_ptr() + a.numel() * a.element_size()
 
 
+def plain(t):
+    """Whether a kernel on t's memory does all that torch operations on t would: no gradient to record, no subclass, no
+    functorch wrapper (vmap, grad, jvp), no forward-mode level, no tracer or dispatch mode that has to see the operations."""
+    return type(t) is torch.Tensor and not t.requires_grad and \
+        not torch._C._functorch.is_functorch_wrapped_tensor(t) and torch.autograd.forward_ad._current_level < 0 and \
+        torch._C._len_torch_dispatch_stack() == 0 and torch._C._get_tracing_state() is None
+
+
+def on_device(t):
+    """Whether t is on the current device, where the kernels of this call are launched."""
+    return t.device.type == "cuda" and t.device.index == torch.cuda.current_device()
+
+
 def stream_buffer(t, dtype, numel, align=16):
-    """Whether t can be read or written by a stream kernel in place: a contiguous device tensor of `dtype` with exactly
-    `numel` elements and an aligned address."""
-    return t.device.type == "cuda" and t.dtype == dtype and t.is_contiguous() and t.numel() == numel and \
+    """Whether t can be read or written by a stream kernel in place: a plain contiguous tensor of `dtype` on the current
+    device with exactly `numel` elements and an aligned address."""
+    return on_device(t) and t.dtype == dtype and plain(t) and t.is_contiguous() and t.numel() == numel and \
         t.data_ptr() % align == 0
 
 

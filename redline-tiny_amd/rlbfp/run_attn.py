@@ -205,7 +205,7 @@ def _tile_range(buf, heads, t_all, t0, n, per=1):
 def _a_buffer(out, rows_all, cols_all):
     """Whether `out` can be written in place as the A-layout stream of a (rows_all, cols_all) matrix (a longer buffer
     may hold more rows)."""
-    return out.device.type == "cuda" and out.dtype == torch.uint8 and out.is_contiguous() and \
+    return ops.on_device(out) and out.dtype == torch.uint8 and ops.plain(out) and out.is_contiguous() and \
         out.data_ptr() % 16 == 0 and rows_all % 128 == 0 and cols_all % 64 == 0 and \
         out.numel() >= ops.packed_bytes(rows_all, cols_all) and out.numel() % 9 == 0
 

@@ -193,10 +193,13 @@ class LM:
             self.tabs[i] = run_qkv.qkv_tables(cos, sin, bf(torch.as_tensor(wq).cuda() * C_LOG2),
                                               torch.as_tensor(wk).cuda()).reshape(-1)
 
+    def _hp_in_place(self):
+        return self.hp_kernel and self.hp.dim() == 1 and ops.stream_buffer(self.hp, torch.int64, self.d, 8)
+
     def load_x(self, x):
         """x (rows, hidden) in the model's channel order; stored in the packed weights' order (:363-366)."""
         x = torch.as_tensor(x, device=self.hp.device)
-        if self.hp_kernel and x.dim() == 2 and x.shape[0] <= self.m and x.shape[1] == self.d:
+        if self._hp_in_place() and x.dim() == 2 and x.shape[0] <= self.m and x.shape[1] == self.d and ops.plain(x):
             x = (x if x.dtype == torch.bfloat16 else x.float()).contiguous()
             if x.data_ptr() % 16:
                 x = x.clone()
@@ -253,7 +256,7 @@ class LM:
         self.queue = True
         try:
             self._rms(x0, self.br, self.br16, self.wts.p_in[last_i], x1, self.a1)
-            if self.hp_kernel:
+            if self._hp_in_place():
                 return ops.stream_unpack(x1, self.m, self.d, perm=self.hp, dtype=torch.float32)
         finally:
             self._settle()
