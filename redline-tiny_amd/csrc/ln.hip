@@ -43,6 +43,23 @@ struct LnArgs {
   int32_t rows_wg;  // rows per workgroup: 4, or 16 for the A-layout order
 };
 
+template <bool NT>
+__device__ __forceinline__ void store_x(uint16_t* p, u32x4 v) {
+  if constexpr (NT)
+    store_stream(p, v);
+  else
+    *reinterpret_cast<u32x4*>(p) = v;
+}
+
+// Whether x' goes past the caches (br: 0 no branch, 1 bf16, 2 packed). It pays where x and the branch are more than the
+// L2s hold (8 x 4 MB): cached x' then pushes out what is still to be read. Cached against past the caches, us, by bytes
+// read: 37 MB (2624 x 3520, bf16 branch) 15.3 / 15.7; 36 MB (4352 x 4096, no branch) 21.1 / 21.6; 42 MB (4352 x 3072,
+// packed) 19.7 / 18.4; 48 MB (4352 x 3520, packed) 24.4 / 22.3; 61 MB (same, bf16) 28.1 / 23.5; 71 MB (8704 x 4096, no
+// branch) 46.6 / 43.0; from 110 MB on the same. On streams (below) it cost nothing at any size, so there it is always so.
+static bool past_caches(int64_t M, int64_t D, int br) {
+  return M * D * (br == 0 ? 16 : br == 1 ? 32 : 25) / 8 > 40000000;
+}
+
 template <int CTRL>
 __device__ __forceinline__ float dpp_f(float x) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xF, 0xF, false));
@@ -78,7 +95,7 @@ template <int NB>
 constexpr int ln_waves_per_simd() { return NB <= 2 ? 6 : NB <= 4 ? 5 : NB <= 6 ? 4 : NB <= 8 ? 3 : NB <= 13 ? 4 : 3; }
 
 // BR: the branch's format for NB <= 8 (0 none, 1 bf16, 2 packed); above 8 blocks it is tested at run time (BR = -1)
-template <int NB, int BR>
+template <int NB, int BR, bool NT>
 __global__ __launch_bounds__(kLnThreads, ln_waves_per_simd<NB>()) void ln_kernel(LnArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t stage[];
   const int lane = threadIdx.x & 63;
@@ -113,7 +130,7 @@ __global__ __launch_bounds__(kLnThreads, ln_waves_per_simd<NB>()) void ln_kernel
         s = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, xw[e]), one, s, false);
       }
       v[j] = u32x4{xw[0], xw[1], xw[2], xw[3]};
-      if (a.x_out) store_stream(a.x_out + r * a.ld_xo + cb * 8, v[j]);
+      if (a.x_out) store_x<NT>(a.x_out + r * a.ld_xo + cb * 8, v[j]);
     };
     // a packed branch block from its 12-byte window (block blk starts at byte 9 blk): exact, as from_bfp16
     auto branch_block = [&](int64_t blk, uint32_t w0, uint32_t w1, uint32_t w2, float (&bf)[8]) {
@@ -265,30 +282,36 @@ __global__ __launch_bounds__(kLnThreads, ln_waves_per_simd<NB>()) void ln_kernel
   }
 }
 
-template <int NB, int BR>
+template <int NB, int BR, bool NT>
 static int launch_nb_br(const LnArgs& a, hipStream_t st) {
   const int64_t lds = a.a_packed ? (int64_t)a.rows_wg * (a.D / 8) * kBlockBytes : 0;
   if (lds > 65536) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&ln_kernel<NB, BR>),
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&ln_kernel<NB, BR, NT>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     if (e != hipSuccess) return fail(RL_ERR_DEVICE, "hipFuncSetAttribute: %s", hipGetErrorString(e));
   }
   const dim3 grid((unsigned)((a.M + a.rows_wg - 1) / a.rows_wg));
-  hipLaunchKernelGGL((ln_kernel<NB, BR>), grid, dim3(kLnThreads), (unsigned)lds, st, a);
+  hipLaunchKernelGGL((ln_kernel<NB, BR, NT>), grid, dim3(kLnThreads), (unsigned)lds, st, a);
   return launch_status("rl_ln_modulate");
 }
 
 // the branch's format is a template parameter, so that the first pass is straight-line code whose loads all issue
 // before the first use
+template <int NB, bool NT>
+static int launch_nb_nt(const LnArgs& a, hipStream_t st) {
+  if constexpr (NB > 8) {
+    return launch_nb_br<NB, -1, NT>(a, st);
+  } else {
+    if (!a.br) return launch_nb_br<NB, 0, NT>(a, st);
+    if (a.br_fmt == RL_BRANCH_BF16) return launch_nb_br<NB, 1, NT>(a, st);
+    return launch_nb_br<NB, 2, NT>(a, st);
+  }
+}
+
 template <int NB>
 static int launch_nb(const LnArgs& a, hipStream_t st) {
-  if constexpr (NB > 8) {
-    return launch_nb_br<NB, -1>(a, st);
-  } else {
-    if (!a.br) return launch_nb_br<NB, 0>(a, st);
-    if (a.br_fmt == RL_BRANCH_BF16) return launch_nb_br<NB, 1>(a, st);
-    return launch_nb_br<NB, 2>(a, st);
-  }
+  const int br = !a.br ? 0 : a.br_fmt == RL_BRANCH_BF16 ? 1 : 2;
+  return a.x_out && past_caches(a.M, a.D, br) ? launch_nb_nt<NB, true>(a, st) : launch_nb_nt<NB, false>(a, st);
 }
 
 template <int NB>

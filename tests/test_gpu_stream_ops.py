@@ -244,3 +244,23 @@ def test_attention_deterministic_on_cold_caches(dev, H, N):
     for i in range(12):
         big.add_(1)
         assert torch.equal(ops.attention(q, k, vt, split=False), ref), i
+
+
+@pytest.mark.parametrize("M,D,branch,packed", [(6600, 3072, "none", False), (3300, 3072, "bf16", True),
+                                               (4300, 3008, "packed", False), (3250, 4096, "packed", True),
+                                               (2600, 4096, "bf16", False), (1300, 8192, "bf16", True),
+                                               (1650, 8192, "packed", False)])
+def test_ln_x_past_the_caches(dev, M, D, branch, packed):
+    """x' stored past the caches (more than 40 MB read): the same bits as from two halves, which are below that line and
+    store it through the caches."""
+    g = torch.Generator(device=dev).manual_seed(M + D)
+    x, b = (torch.randn(M, D, device=dev, generator=g).to(torch.bfloat16) for _ in range(2))
+    params = torch.randn(2, 2 * D, device=dev, generator=g).to(torch.bfloat16)
+    br = lambda r: {"none": None, "bf16": b[r], "packed": ops.quantize(b[r].contiguous())[0]}[branch]
+    run = lambda r: ops.ln_modulate(x[r], params, branch=br(r), norm="layer", packed=packed, deq=True)
+    whole, h = run(slice(0, M)), M // 2
+    lo, hi = run(slice(0, h)), run(slice(h, M))
+    assert torch.equal(whole[0], torch.cat([lo[0], hi[0]]))
+    assert torch.equal(whole[2], torch.cat([lo[2], hi[2]]))
+    if packed:
+        assert torch.equal(whole[1].reshape(-1), torch.cat([lo[1].reshape(-1), hi[1].reshape(-1)]))
